@@ -1,0 +1,49 @@
+"""The FP32 kernels' products on the bf16 matrix cores (six term products of
+the three-term splits, TraitsX6), against FP64 at FP32's own error bound.
+
+One year with the pre-growth endpoint returns the product itself.  With K
+terms a destination's value takes ceil(K / 8) roundings of the sum of the
+large term products and as many, 2^-8 smaller, of the small ones (each
+rounding cut by at most 2^-8 of the last place), one rounding each of the
+state, the movement entry and the final sum, and the dropped term products:
+|error| <= (ceil(K / 8) (1 + 2^-6) + 6) 2^-24 of a sum of non-negative terms.
+A product without any one of the six terms exceeds it."""
+import numpy as np
+import pytest
+
+from transportoptimiser_amd import landscape as ls
+from transportoptimiser_amd import native as nat
+
+pytestmark = pytest.mark.gpu
+
+# Patch counts around the 16-term chunks, the 32-wide tiles and the waves'
+# shares; path counts that make one, two, three (single row tiles) and more
+# row tiles, whole and ragged.
+SIZES = [1, 15, 16, 17, 31, 33, 48, 64, 65, 96, 130, 160, 200, 257, 300, 416, 512, 700, 1024]
+
+
+def _road(P, N, seed):
+    rng = np.random.default_rng([seed, P, N])
+    # Populations over six decades and entries over nine: every term of the
+    # splits, and sums led by one product, count.
+    init = 10.0 ** rng.uniform(-3, 3, P)
+    trans = 10.0 ** rng.uniform(-9, 0, (P, P))
+    trans /= trans.sum(1, keepdims=True)
+    surv = 1.0 - rng.uniform(0.0, 0.5, (P, P))
+    sd = ls.SpeciesData(trans=np.asfortranarray(trans), surv=np.asfortranarray(surv),
+                        init_pop=init, capacity=np.full(P, 1e4), growth=np.zeros(P))
+    return ls.RoadProblem([sd], n_years=1, n_paths=N, endpoint=nat.END_PRE_GROWTH, seed=seed)
+
+
+@pytest.mark.parametrize("N", [1, 70, 256, 300])
+def test_one_year_product_within_the_fp32_bound(ctx, N):
+    for P in SIZES:
+        pr = _road(P, N, 3)
+        sd = pr.species[0]
+        print(f"P={P} N={N}", flush=True)
+        ref = (sd.init_pop[:, None] * sd.trans * sd.surv).sum(0)
+        bound = (-(-P // 8) * (1 + 2.0 ** -6) + 6) * 2.0 ** -24
+        for out in (ctx.simulate_mte(pr), ctx.simulate_mte_batch([pr], end_pops=True)[0]):
+            err = np.abs(out.patch_mean[0] - ref) / ref
+            assert err.max() <= bound, (P, err.max(), bound)
+            np.testing.assert_allclose(out.end_pops[:, 0], ref.sum(), rtol=bound)

@@ -90,7 +90,7 @@ extern "C" void roadmc_ctx_destroy(roadmc_ctx* ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
-  rmc_devbuf* bufs[] = {&ctx->mte_bufs.mpack, &ctx->mte_bufs.cols, &ctx->mte_bufs.partial,
+  rmc_devbuf* bufs[] = {&ctx->mte_bufs.mpack, &ctx->mte_bufs.mx6,  &ctx->mte_bufs.cols, &ctx->mte_bufs.partial,
                         &ctx->mte_bufs.out,   &ctx->mte_bufs.endpop, &ctx->mte_bufs.jobs,
                         &ctx->mte_bufs.work,  &ctx->mte_bufs.off,  &ctx->mte_bufs.counter,
                         &ctx->rov_bufs.a,     &ctx->rov_bufs.b,    &ctx->rov_bufs.c,

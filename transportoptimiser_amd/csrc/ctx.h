@@ -15,7 +15,9 @@ struct rmc_devbuf {
 };
 
 struct rmc_job_buffers {
-  rmc_devbuf mpack, cols, partial, out, endpop, jobs, work, off, counter;
+  // mpack: the packed movement matrices as uploaded or built; mx6: their
+  // three-term split (FP32 launches).
+  rmc_devbuf mpack, mx6, cols, partial, out, endpop, jobs, work, off, counter;
 };
 
 struct roadmc_ctx {

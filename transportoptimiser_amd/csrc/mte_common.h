@@ -125,6 +125,94 @@ struct TraitsB3 {
   }
 };
 
+// FP32 products on v_mfma_f32_32x32x16_bf16.  An FP32 value is exactly the sum
+// of three bf16 terms x = h + m + l (each the rounding of what is left), and a
+// product x.y is taken as the six of the nine term products that reach 2^-24
+// of it: h.h' in one FP32 accumulator, l.h' + h.l' + m.m' + m.h' + h.m' in a
+// second one, added to the first at the end.  The dropped m.l', l.m' and l.l'
+// are below 2^-25 of the product, of either sign.
+// Why two accumulators: the matrix cores add 8 products at a time (their sum
+// aligned to the largest one's exponent - 24) to the accumulator and round to
+// nearest, but cut the sum to 2^-8 of the accumulator's last place, downwards.
+// In one accumulator, twelve such cuts per 16 products lower every sum by
+// 2e-8 of it at 256 terms, each year alike; in two the bias is below 1e-9 and
+// the rms error of a dot product over landscape rows is less than half that
+// of v_mfma_f32_32x32x2_f32 (5.1e-8 against 1.2e-7 at 64 terms, 9.1e-8
+// against 2.3e-7 at 256, 1.8e-7 against 4.8e-7 at 1024).
+// The matrix cores run the six at 1.8 PFLOP/s (random operands), 305 TFLOP/s
+// of FP32 products against 155 for the FP32 MFMA, and leave the VALU to the
+// other waves of the SIMD, which the FP32 MFMA does not.
+// The population tile stays FP32 in LDS, k in natural order, and is split as
+// it is read (28 VALU operations per 8 values); the movement matrix is split
+// once when it is packed.  Operand and accumulator lane layouts are those of
+// TraitsB3.
+struct TraitsX6 {
+  using T = float;
+  using VecT = floatx4;
+  using AccT = floatx16;
+  static constexpr int TM = 32, TN = 32, KV = 8, NACC = 16, NT = 4, PAD = 4;
+  static constexpr bool kQuadItems = true;
+  static constexpr bool kSplit = false;
+  __device__ static AccT mfma(floatx4 a, floatx4 b, AccT c) { return TraitsB3::mfma(a, b, c); }
+  __device__ static int acc_row(int lane, int r) {
+    return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+  }
+  __device__ static int acc_col(int lane) { return lane & 31; }
+  __device__ static int a_row(int lane) { return lane & 31; }
+  __device__ static int k_lane(int lane) { return lane >> 5; }
+  __host__ __device__ static int perm(int k) { return k; }
+  __device__ static float expo(float x) { return __expf(x); }
+  __device__ static void normal4(uint32_t q, uint32_t y, uint32_t p,
+                                 uint32_t tag, uint32_t k0, uint32_t k1,
+                                 float z[4]) {
+    rmc_normal4_f(q, y, p, tag, k0, k1, z);
+  }
+};
+
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// The three bf16 terms of a pair of FP32 values, packed (first value in the
+// low half), each the rounding to nearest of what the ones before leave, so
+// that m and l have either sign and h + m + l is the value.  x - h is one v_dot2_f32_bf16 of the
+// packed pair with (-1, 0) or (0, -1), exact because the difference is
+// representable; the constants stay in scalar registers (as inline constants
+// they would read as a 32-bit -1.0).
+__device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& h, uint32_t& m,
+                                            uint32_t& l) {
+  uint32_t c0 = 0x0000bf80u, c1 = 0xbf800000u;
+  asm("" : "+s"(c0), "+s"(c1));
+  const bf16x2 n0 = __builtin_bit_cast(bf16x2, c0), n1 = __builtin_bit_cast(bf16x2, c1);
+  auto pack = [](float a, float b) -> uint32_t {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){a, b}, bf16x2));
+  };
+  auto minus = [](uint32_t pk, bf16x2 which, float x) -> float {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pk), which, x, false);
+  };
+  h = pack(x0, x1);
+  const float r0 = minus(h, n0, x0), r1 = minus(h, n1, x1);
+  m = pack(r0, r1);
+  l = pack(minus(m, n0, r0), minus(m, n1, r1));
+}
+
+// The split operands of 8 consecutive FP32 values.
+struct Split8 {
+  floatx4 h, m, l;
+};
+__device__ __forceinline__ Split8 split3_8(const floatx4 x0, const floatx4 x1) {
+  uint32_t h[4], m[4], l[4];
+  split3_pair(x0[0], x0[1], h[0], m[0], l[0]);
+  split3_pair(x0[2], x0[3], h[1], m[1], l[1]);
+  split3_pair(x1[0], x1[1], h[2], m[2], l[2]);
+  split3_pair(x1[2], x1[3], h[3], m[3], l[3]);
+  typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
+  Split8 s;
+  s.h = __builtin_bit_cast(floatx4, (uint32x4){h[0], h[1], h[2], h[3]});
+  s.m = __builtin_bit_cast(floatx4, (uint32x4){m[0], m[1], m[2], m[3]});
+  s.l = __builtin_bit_cast(floatx4, (uint32x4){l[0], l[1], l[2], l[3]});
+  return s;
+}
+
 __host__ __device__ static inline size_t align16(size_t x) {
   return (x + 15) & ~(size_t)15;
 }
@@ -447,6 +535,77 @@ __device__ __forceinline__ void range_product_b3(floatx16& acc, const PackedB& B
     products(ah1, al1, bh1, bl1);
   }
   if (c < c1) products(ah0, al0, bh0, bl0);
+}
+
+// Byte offset of lane `lane`'s operands of column block `tcol` in a matrix
+// packed for TraitsX6 (nch 16-k chunks, each 3 x 1 KB: the h, m and l
+// operands of the 64 lanes).
+__device__ __forceinline__ uint32_t b6_voff(int nch, int tcol, int lane) {
+  return ((uint32_t)tcol * (uint32_t)nch * 192u + (uint32_t)lane) * 16u;
+}
+
+// acc[c * NR + r] = A[row tile r, chunks c0 .. c1) . M[those chunks, column
+// tile c] for NR row tiles x NC column tiles (TraitsX6), c1 > c0; ap is the
+// lane's first operand of row tile 0 (chunk 0), rstep the row tiles' distance
+// and boff[c] the column tiles' offsets.  Blocks of 2 x 2 tiles use each split
+// and each B operand for two tiles: 14 VALU operations and 1.5 KB of L2
+// traffic per six MFMAs, against 28 and 3 KB for single tiles.  The B operands
+// of the next chunk are in flight while this chunk's products run; the A
+// operands are split first, then reloaded for the next chunk.
+template <int NR, int NC>
+__device__ __forceinline__ void product_x6(floatx16* acc, const PackedB& B, const float* ap,
+                                           int rstep, const uint32_t* boff, int c0, int c1) {
+  floatx16 sm[NR * NC];
+#pragma unroll
+  for (int t = 0; t < NR * NC; ++t) acc[t] = sm[t] = floatx16{};
+  floatx4 b0[NC][3], b1[NC][3], a[NR][2];
+  auto ldb = [&](floatx4 (&b)[NC][3], int c) {
+#pragma unroll
+    for (int t = 0; t < NC; ++t)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) b[t][i] = load_b<floatx4>(B, boff[t], 3 * c + i);
+  };
+  auto lda = [&](int c) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const floatx4* q = reinterpret_cast<const floatx4*>(ap + r * rstep + 16 * c);
+      a[r][0] = q[0];
+      a[r][1] = q[1];
+    }
+  };
+  auto step = [&](const floatx4 (&b)[NC][3], floatx4 (&bn)[NC][3], const int c) {
+    const int cn = min(c + 1, c1 - 1);
+    ldb(bn, cn);
+    Split8 x[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) x[r] = split3_8(a[r][0], a[r][1]);
+    lda(cn);
+    // Keep the loads ahead of the products, which do not need them.
+    __builtin_amdgcn_sched_barrier(0);
+    // One term product at a time over the tiles, so that consecutive MFMAs
+    // are independent.
+#define RMC_X6(d, ta, ib)                                                      \
+  _Pragma("unroll") for (int t = 0; t < NC; ++t)                               \
+      _Pragma("unroll") for (int r = 0; r < NR; ++r) d[t * NR + r] =           \
+          TraitsX6::mfma(x[r].ta, b[t][ib], d[t * NR + r])
+    RMC_X6(sm, l, 0);
+    RMC_X6(sm, h, 2);
+    RMC_X6(sm, m, 1);
+    RMC_X6(sm, m, 0);
+    RMC_X6(sm, h, 1);
+    RMC_X6(acc, h, 0);
+#undef RMC_X6
+  };
+  ldb(b0, c0);
+  lda(c0);
+  int c = c0;
+  for (; c + 1 < c1; c += 2) {
+    step(b0, b1, c);
+    step(b1, b0, c + 1);
+  }
+  if (c < c1) step(b0, b1, c);
+#pragma unroll
+  for (int t = 0; t < NR * NC; ++t) acc[t] += sm[t];
 }
 
 }  // namespace roadmc

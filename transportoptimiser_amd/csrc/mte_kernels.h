@@ -15,7 +15,8 @@ enum { kPrecF32 = 0, kPrecF64 = 1, kPrecB3 = 2 };
 // One (road, species) pair of a launch.  Device arrays are of the launch's
 // element type (float for FP32, double for FP64).
 struct MteJob {
-  const void* mpack;   // movement matrix in MFMA B-operand order, Pp*Pp
+  const void* mpack;   // movement matrix in MFMA B-operand order, Pp*Pk (FP32:
+                       // its three-term split, 6 bytes an entry)
   const void* cols;    // 4*Pp: capacity, 1/capacity, growth rate, initial pop
   double* end_pops;    // [N] per-path end totals, or nullptr
   void* ckpt;          // adjoint checkpoints [T/ckpt_every][N][Pp], or nullptr
@@ -70,6 +71,10 @@ int mte_tiles_per_wave(int prec, int BM, int Pp);
 hipError_t mte_set_lds_limit(int prec, size_t bytes);
 hipError_t launch_mte_direct(int prec, int tiles_per_wave, const MteJob* jobs,
                              const int2* work, int n_work, size_t lds, hipStream_t s);
+// Splits FP32-packed matrices (n_floats, a multiple of 512) into the
+// three-term operands the FP32 kernels take: 1.5 n_floats floats at out, each
+// matrix at 1.5 times its offset.
+hipError_t launch_mte_split_x6(const float* m, size_t n_floats, float* out, hipStream_t s);
 // Converts FP32-packed matrices (n_floats, a multiple of 512, each matrix
 // with an even k-group count) in place to the split-bf16 operand order.
 hipError_t launch_mte_split_b3(float* m, size_t n_floats, hipStream_t s);

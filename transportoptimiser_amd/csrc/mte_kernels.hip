@@ -16,8 +16,8 @@
 //     for 4 consecutive k-steps are one 16-byte LDS read;
 //   - R is pre-packed in MFMA B-operand order, so each wave's B load is one
 //     coalesced 1 KB read that L2 serves to every workgroup of the road;
-//   - products run on v_mfma_f32_32x32x2_f32 (FP32 accumulate) or, for the
-//     FP64 checker path, v_mfma_f64_16x16x4_f64;
+//   - FP32 products run as six bf16 term products (TraitsX6, FP32 accumulate)
+//     and, for the FP64 checker path, on v_mfma_f64_16x16x4_f64;
 //   - the epilogue draws the year noise from counter-based Philox in
 //     registers (no random arrays in HBM), applies the growth law, and writes
 //     the new population back to LDS; after the last year it reduces the
@@ -39,7 +39,7 @@ size_t mte_lds_bytes(int prec, int BM, int Pp, int n_rem_split) {
   switch (prec) {
     case kPrecF64: return lds_bytes_t<TraitsF64>(BM, Pp, n_rem_split);
     case kPrecB3: return lds_bytes_t<TraitsB3>(BM, Pp, n_rem_split);
-    default: return lds_bytes_t<TraitsF32>(BM, Pp, n_rem_split);
+    default: return lds_bytes_t<TraitsX6>(BM, Pp, n_rem_split);
   }
 }
 
@@ -58,6 +58,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   using VecT = typename TR::VecT;
   using AccT = typename TR::AccT;
   constexpr int TM = TR::TM, TN = TR::TN, KV = TR::KV, NACC = TR::NACC;
+  constexpr bool kX6 = std::is_same<TR, TraitsX6>::value;
   const int tid = threadIdx.x, lane = tid & 63;
   // Wave index as a scalar: the per-wave tile loops below then branch on
   // SGPRs instead of exec masks.
@@ -131,20 +132,30 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   const int my_np = upper ? n_rem : 0;  // k-quarter pieces of this wave
   T* qpart = reinterpret_cast<T*>(reinterpret_cast<char*>(red) + 8 * 4 * sizeof(double));
   int trow[NT], tcol[NT];
+  // Where the FP32 form has an even number of row tiles, tiles are numbered
+  // down pairs of row tiles (both tiles of a column, then the next column), so
+  // that a wave's run of tiles is made of 2 x 2 and 2 x 1 blocks.
+  const bool row_pairs = kX6 && ((BM / TM) & 1) == 0;
+  auto tile_pos = [&](const int ti, int& tr, int& tc) {
+    if (row_pairs) {
+      const int g = ti / (2 * ntc), rem = ti - g * 2 * ntc;
+      tr = 2 * g + (rem & 1);
+      tc = rem >> 1;
+    } else {
+      tr = ti / ntc;
+      tc = ti - tr * ntc;
+    }
+  };
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int ti = my_t0 + t;
-    trow[t] = ti / ntc;
-    tcol[t] = ti - (ti / ntc) * ntc;
-  }
+  for (int t = 0; t < NT; ++t) tile_pos(my_t0 + t, trow[t], tcol[t]);
 
   // The contraction runs over Pk = P rounded up to 16 (the packed matrix has
   // Pk / 8 k-groups); output columns run over Pp = P rounded up to 32.
   const int nkg = jb.Pk >> 3;
-  const PackedB Bm = packed_b(jb.mpack, nkg, (size_t)Pp * jb.Pk * sizeof(T));
+  const PackedB Bm = packed_b(jb.mpack, nkg, (size_t)Pp * jb.Pk * (kX6 ? 6 : sizeof(T)));
   // A operand offset of the lane half: KV floats (8 bf16 in the split form).
   const int arow = TR::a_row(lane), akoff = (TR::kSplit ? 8 : KV) * TR::k_lane(lane);
-  const int nch = nkg >> 1;  // split form: 16-k chunks
+  const int nch = nkg >> 1;  // 16-k chunks (the bf16 forms)
 
   // All of this wave's tiles in one row block (contiguous runs usually are):
   // they can share one A fragment per k-group.
@@ -152,7 +163,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
 
   AccT acc[NT];
   VecT b0[NT];
-  if constexpr (!TR::kSplit) {
+  if constexpr (!TR::kSplit && !kX6) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
       if (t < my_n) b0[t] = load_b<VecT>(Bm, b_voff(Bm, tcol[t], lane), 0);
@@ -206,20 +217,74 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
         default: break;
       }
 #undef RMC_YP3
-    } else {
-      // k-quarter pieces of the remainder tiles first (their partial products
-      // go to LDS): the wave with pieces then overlaps its whole tiles with the
-      // other wave on its SIMD instead of finishing alone on a one-tile chain.
+    } else if constexpr (kX6) {
+      // The same schedule: k-quarter pieces first, then the whole tiles in
+      // blocks of 2 x 2, 2 x 1, 1 x 2 or single tiles.
+      const float* const Al = A + arow * LDAy + akoff;
       for (int i = 0; i < my_np; ++i) {
-        const int ti = 4 * q4 + i;
-        const int tr = ti / ntc, tc = ti - (ti / ntc) * ntc;
-        AccT pacc = AccT{};
-        range_product<TR>(pacc, Bm, A, tr, tc, (simd * nkg) >> 2, ((simd + 1) * nkg) >> 2,
-                          LDAy, arow, akoff, lane);
+        int tr, tc;
+        tile_pos(4 * q4 + i, tr, tc);
+        AccT pacc;
+        const uint32_t bo = b6_voff(nch, tc, lane);
+        product_x6<1, 1>(&pacc, Bm, Al + tr * TM * LDAy, 0, &bo, (simd * nch) >> 2,
+                         ((simd + 1) * nch) >> 2);
         T* slot = qpart + (size_t)((i * 4 + simd) * NACC) * 64 + lane;
-  #pragma unroll
+#pragma unroll
         for (int r = 0; r < NACC; ++r) slot[r * 64] = pacc[r];
       }
+      // No value of last year's accumulators lives across the products.
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = AccT{};
+      // Block of NR x NC tiles at tile i of the run.
+      auto block = [&](auto nr, auto nc, auto i) {
+        constexpr int NR = decltype(nr)::value, NC = decltype(nc)::value, I = decltype(i)::value;
+        if constexpr (I + NR * NC <= NT) {
+          uint32_t bo[NC];
+#pragma unroll
+          for (int t = 0; t < NC; ++t) bo[t] = b6_voff(nch, tcol[I + t * NR], lane);
+          product_x6<NR, NC>(acc + I, Bm, Al + trow[I] * TM * LDAy, TM * LDAy, bo, 0, nch);
+        }
+      };
+      using One = std::integral_constant<int, 1>;
+      using Two = std::integral_constant<int, 2>;
+      using I0 = std::integral_constant<int, 0>;
+      using I1 = One;
+      using I2 = Two;
+      using I3 = std::integral_constant<int, 3>;
+      if (row_pairs) {
+        if ((my_t0 & 1) == 0) {
+          if (my_n >= 4 && trow[0] == trow[NT >= 4 ? 2 : 0]) {
+            block(Two{}, Two{}, I0{});
+          } else {
+            if (my_n >= 2) block(Two{}, One{}, I0{});
+            if (my_n == 1) block(One{}, One{}, I0{});
+            if (my_n == 3) block(One{}, One{}, I2{});
+            if (my_n >= 4) block(Two{}, One{}, I2{});
+          }
+        } else {
+          if (my_n >= 1) block(One{}, One{}, I0{});
+          if (my_n >= 3) block(Two{}, One{}, I1{});
+          if (my_n == 2) block(One{}, One{}, I1{});
+          if (my_n >= 4) block(One{}, One{}, I3{});
+        }
+      } else {
+        auto two = [&](auto i) {
+          constexpr int I = decltype(i)::value;
+          if constexpr (I + 2 <= NT) {
+            if (trow[I] == trow[I + 1]) {
+              block(One{}, Two{}, i);
+            } else {
+              block(One{}, One{}, i);
+              block(One{}, One{}, std::integral_constant<int, I + 1>{});
+            }
+          }
+        };
+        if (my_n >= 2) two(I0{});
+        if (my_n == 1) block(One{}, One{}, I0{});
+        if (my_n == 3) block(One{}, One{}, I2{});
+        if (my_n >= 4) two(I2{});
+      }
+    } else {
       // One branch per year on the (wave-uniform) tile count and row sharing;
       // the product loops themselves are straight-line code.
       switch (my_n * 2 + (shared_a ? 1 : 0)) {
@@ -339,8 +404,9 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       for (int qq = 0; qq < 4; ++qq)
 #pragma unroll
         for (int r = 0; r < NACC; ++r) sum[r] += slot[(qq * NACC + r) * 64];
-      const int ti = 4 * q4 + simd;
-      epilogue(sum, ti / ntc, ti - (ti / ntc) * ntc);
+      int tr, tc;
+      tile_pos(4 * q4 + simd, tr, tc);
+      epilogue(sum, tr, tc);
     }
     __syncthreads();
   }
@@ -476,9 +542,9 @@ const void* mte_form(int prec, int tiles_per_wave, bool direct) {
     case kPrecF64: return mte_fn<TraitsF64, TraitsF64::NT>(direct);
     case kPrecB3: return mte_fn<TraitsB3, TraitsB3::NT>(direct);
     default:
-      if (tiles_per_wave <= 1) return mte_fn<TraitsF32, 1>(direct);
-      if (tiles_per_wave <= 2) return mte_fn<TraitsF32, 2>(direct);
-      return mte_fn<TraitsF32, TraitsF32::NT>(direct);
+      if (tiles_per_wave <= 1) return mte_fn<TraitsX6, 1>(direct);
+      if (tiles_per_wave <= 2) return mte_fn<TraitsX6, 2>(direct);
+      return mte_fn<TraitsX6, TraitsX6::NT>(direct);
   }
 }
 
@@ -552,6 +618,34 @@ __global__ __launch_bounds__(64) void mte_split_b3_kernel(float* __restrict__ m)
   uint4* out = reinterpret_cast<uint4*>(c);
   out[l] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
   out[64 + l] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+}
+
+// FP32-packed movement matrices to the operand order of TraitsX6: the
+// 512-float chunk that mte_split_b3_kernel describes becomes 3 KB, lane l's
+// 8 h, m and l terms at bytes 16 l, 1024 + 16 l and 2048 + 16 l.
+__device__ __forceinline__ void split_x6_chunk(const RMC_GLOBAL float* c, float* out) {
+  const int l = threadIdx.x & 63, n = l & 31, g = l >> 5;
+  floatx4 v[2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i >> 2][i & 3] = c[(64 * g + 32 * (i & 1) + n) * 4 + (i >> 1)];
+  const Split8 s = split3_8(v[0], v[1]);
+  floatx4* o = reinterpret_cast<floatx4*>(out);
+  o[l] = s.h;
+  o[64 + l] = s.m;
+  o[128 + l] = s.l;
+}
+
+__global__ __launch_bounds__(64) void mte_split_x6_kernel(const float* __restrict__ m,
+                                                          float* __restrict__ out) {
+  split_x6_chunk(gmem(m) + (size_t)blockIdx.x * 512, out + (size_t)blockIdx.x * 768);
+}
+
+hipError_t launch_mte_split_x6(const float* m, size_t n_floats, float* out, hipStream_t s) {
+  if (n_floats % 512 != 0) return hipErrorInvalidValue;
+  if (n_floats == 0) return hipSuccess;
+  hipLaunchKernelGGL(mte_split_x6_kernel, dim3((unsigned)(n_floats / 512)), dim3(64), 0, s, m,
+                     out);
+  return hipGetLastError();
 }
 
 hipError_t launch_mte_split_b3(float* m, size_t n_floats, hipStream_t s) {

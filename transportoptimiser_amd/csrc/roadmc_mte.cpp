@@ -330,7 +330,9 @@ int upload_jobs(roadmc_ctx* ctx, const roadmc_mte_problem* roads, JobSet& js,
     return persistent_bufs ? rmc_buf_alloc_exact(ctx, buf, bytes)
                            : rmc_buf_ensure(ctx, buf, bytes);
   };
+  const bool x6 = js.prec == roadmc::kPrecF32;
   if ((rc = grow(b.mpack, js.mpack_elems * es)) ||
+      (x6 && (rc = grow(b.mx6, js.mpack_elems * 6))) ||
       (rc = grow(b.cols, js.cols_elems * es)) ||
       (rc = grow(b.partial, js.part_elems * sizeof(double))) ||
       (rc = grow(b.out, js.out_elems * sizeof(double))) ||
@@ -377,7 +379,8 @@ int upload_jobs(roadmc_ctx* ctx, const roadmc_mte_problem* roads, JobSet& js,
   }
   for (size_t j = 0; j < nj; ++j) {
     MteJob& jb = js.jobs[j];
-    jb.mpack = static_cast<T*>(b.mpack.ptr) + js.mpack_off[j];
+    jb.mpack = x6 ? static_cast<void*>(static_cast<char*>(b.mx6.ptr) + js.mpack_off[j] * 6)
+                  : static_cast<void*>(static_cast<T*>(b.mpack.ptr) + js.mpack_off[j]);
     jb.cols = static_cast<T*>(b.cols.ptr) + js.cols_off[j];
     jb.partial = static_cast<double*>(b.partial.ptr) + js.part_off[j];
     jb.end_pops = js.endpop_off[j] >= 0
@@ -457,7 +460,11 @@ int upload_jobs(roadmc_ctx* ctx, const roadmc_mte_problem* roads, JobSet& js,
       RMC_HIP(ctx, hipStreamWaitEvent(s, l.done, 0));
     }
   }
-  // Split-bf16 operands are converted in place from the FP32 packing.
+  // The bf16 operands are converted from the FP32 packing: the three-term
+  // split of the FP32 kernels, the two-term split in place.
+  if (x6)
+    RMC_HIP(ctx, roadmc::launch_mte_split_x6(static_cast<float*>(b.mpack.ptr), js.mpack_elems,
+                                             static_cast<float*>(b.mx6.ptr), s));
   if (js.prec == roadmc::kPrecB3)
     RMC_HIP(ctx, roadmc::launch_mte_split_b3(static_cast<float*>(b.mpack.ptr), js.mpack_elems, s));
   roadmc::RoadTail tail{0, {0, 0, 0}};
@@ -897,7 +904,7 @@ extern "C" void roadmc_batch_destroy(roadmc_batch* bt) {
   }
   if (bt->exec) (void)hipGraphExecDestroy(bt->exec);
   if (bt->graph) (void)hipGraphDestroy(bt->graph);
-  rmc_devbuf* all[] = {&bt->bufs.mpack, &bt->bufs.cols, &bt->bufs.partial, &bt->bufs.out,
+  rmc_devbuf* all[] = {&bt->bufs.mpack, &bt->bufs.mx6, &bt->bufs.cols, &bt->bufs.partial, &bt->bufs.out,
                        &bt->bufs.endpop, &bt->bufs.jobs, &bt->bufs.work, &bt->bufs.off,
                        &bt->bufs.counter};
   for (rmc_devbuf* d : all) rmc_buf_free(*d);
@@ -1347,6 +1354,11 @@ int adjoint_upload(roadmc_adjoint* adj, const roadmc_species& sp, double tol) {
     return rc;
   RMC_HIP(ctx, hipMemcpy(adj->bufs.mpack.ptr, mp.data(), mp.size() * sizeof(T),
                          hipMemcpyHostToDevice));
+  if (!fp64) {
+    if ((rc = rmc_buf_alloc_exact(ctx, adj->bufs.mx6, mp.size() * 6))) return rc;
+    RMC_HIP(ctx, roadmc::launch_mte_split_x6(static_cast<float*>(adj->bufs.mpack.ptr), mp.size(),
+                                             static_cast<float*>(adj->bufs.mx6.ptr), ctx->stream));
+  }
   RMC_HIP(ctx, hipMemcpy(adj->mtpack.ptr, mt.data(), mt.size() * sizeof(T),
                          hipMemcpyHostToDevice));
   RMC_HIP(ctx, hipMemcpy(adj->bufs.cols.ptr, cols.data(), cols.size() * sizeof(T),
@@ -1367,7 +1379,7 @@ extern "C" void roadmc_adjoint_destroy(roadmc_adjoint* adj) {
     spare = adj->ckpt;
     adj->ckpt = rmc_devbuf{};
   }
-  rmc_devbuf* all[] = {&adj->bufs.mpack, &adj->bufs.cols, &adj->bufs.partial, &adj->bufs.out,
+  rmc_devbuf* all[] = {&adj->bufs.mpack, &adj->bufs.mx6, &adj->bufs.cols, &adj->bufs.partial, &adj->bufs.out,
                        &adj->bufs.endpop, &adj->bufs.jobs, &adj->bufs.work, &adj->bufs.off,
                        &adj->bufs.counter, &adj->mtpack, &adj->ckpt};
   for (rmc_devbuf* d : all) rmc_buf_free(*d);
@@ -1445,7 +1457,7 @@ extern "C" int roadmc_mte_adjoint_fwd(roadmc_ctx* ctx, const roadmc_mte_problem*
     roadmc_adjoint_destroy(adj);
     return rc;
   }
-  jb.mpack = adj->bufs.mpack.ptr;
+  jb.mpack = adj->fp64 ? adj->bufs.mpack.ptr : adj->bufs.mx6.ptr;
   jb.cols = adj->bufs.cols.ptr;
   jb.partial = static_cast<double*>(adj->bufs.partial.ptr);
   jb.end_pops = nullptr;
