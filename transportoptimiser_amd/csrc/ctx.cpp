@@ -123,6 +123,9 @@ extern "C" void roadmc_ctx_destroy(roadmc_ctx* ctx) {
     if (l.stream) (void)hipStreamDestroy(l.stream);
   }
   if (ctx->road_ready) (void)hipEventDestroy(ctx->road_ready);
+  if (ctx->batch_fork) (void)hipEventDestroy(ctx->batch_fork);
+  if (ctx->batch_join) (void)hipEventDestroy(ctx->batch_join);
+  if (ctx->batch_side) (void)hipStreamDestroy(ctx->batch_side);
   if (ctx->pinned) (void)hipHostFree(ctx->pinned);
   if (ctx->rov_graph.exec) (void)hipGraphExecDestroy(ctx->rov_graph.exec);
   rmc_buf_free(ctx->rov_graph.param);

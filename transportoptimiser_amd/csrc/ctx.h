@@ -35,7 +35,7 @@ struct roadmc_ctx {
   struct TileSetting {
     int rows, split, per_cu;
   };
-  TileSetting tiles[2][4] = {{{256, 1, 0}, {128, 1, 0}, {64, 1, 0}, {32, 1, 0}},
+  TileSetting tiles[2][4] = {{{128, 1, 0}, {64, 1, 0}, {64, 1, 0}, {32, 1, 0}},
                              {{256, 1, 0}, {128, 1, 0}, {64, 1, 0}, {32, 1, 0}}};
   rmc_job_buffers mte_bufs;
   struct {
@@ -74,6 +74,10 @@ struct roadmc_ctx {
     rmc_devbuf cross, trans, surv, blockmax, part;
   } road_lanes[kRoadLanes];
   hipEvent_t road_ready = nullptr;
+  // Side stream (default priority) of the second launch of a batch's graph
+  // and the events that fork and join it; created on first use.
+  hipStream_t batch_side = nullptr;
+  hipEvent_t batch_fork = nullptr, batch_join = nullptr;
   // Pinned host staging of the packed operands (grown on demand, kept).
   void* pinned = nullptr;
   size_t pinned_bytes = 0;

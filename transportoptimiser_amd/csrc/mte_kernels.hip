@@ -50,8 +50,8 @@ size_t mte_lds_bytes(int prec, int BM, int Pp, int n_rem_split) {
 // NT bounds the output tiles per wave: the accumulators and operands of NT
 // tiles are allocated whether or not a wave uses them, so the launch picks the
 // smallest form that holds its jobs' tiles, which leaves registers for more
-// resident workgroups.
-template <class TR, int LAW, int NT>
+// resident workgroups.  NW is the workgroup's waves.
+template <class TR, int LAW, int NT, int NW>
 __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
                                              char* smem) {
   using T = typename TR::T;
@@ -63,7 +63,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   // Wave index as a scalar: the per-wave tile loops below then branch on
   // SGPRs instead of exec masks.
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nthreads = blockDim.x, nwaves = nthreads >> 6;
+  constexpr int nthreads = NW * 64, nwaves = NW;
   const int BM = jb.BM, Pp = jb.Pp, LDA = Pp + TR::PAD;
   const int p0 = tile * BM;
 
@@ -104,32 +104,33 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   __syncthreads();
 
   // Output tiles (TM x TN blocks of the BM x Pp result) and who computes
-  // them.  Waves w and w + 4 run on the same SIMD, so the work that has to be
-  // even is each SIMD's, not each wave's.
+  // them.  Waves w, w + 4, ... run on the same SIMD, so the work that has to
+  // be even is each SIMD's, not each wave's.
   //  - Without splitting: wave w takes a contiguous run of ceil or floor of
-  //    ntiles / 8 tiles.
-  //  - With splitting (jb.split): each SIMD takes q = ntiles / 4 whole tiles
-  //    (ceil(q/2) in wave s, the rest in wave s + 4), and each of the
-  //    ntiles % 4 remaining tiles is cut into four k-quarters, quarter s going
-  //    to wave s + 4.  The quarters meet in LDS, where wave i + 4 sums the four
-  //    partial products of remainder tile i in a fixed order and applies its
-  //    epilogue.
+  //    ntiles / NW tiles.
+  //  - With splitting (jb.split): each SIMD takes q = ntiles / 4 whole tiles,
+  //    shared evenly by its waves, and each of the ntiles % 4 remaining tiles
+  //    is cut into four k-quarters, quarter s going to the last wave of SIMD
+  //    s.  The quarters meet in LDS, where the last wave of SIMD i sums the
+  //    four partial products of remainder tile i in a fixed order and applies
+  //    its epilogue.
   const int ntc = Pp / TN;
   const int ntiles = (BM / TM) * ntc;
-  const int simd = wave & 3, upper = wave >> 2;
+  const int simd = wave & 3, nth = wave >> 2;
+  const bool pieces = nth == NW / 4 - 1;  // takes the k-quarter pieces
   int my_n, my_t0, n_rem = 0, q4 = 0;
   if (jb.split) {
     q4 = ntiles >> 2;
     n_rem = ntiles & 3;
-    const int qa = (q4 + 1) >> 1;
-    my_n = upper ? q4 - qa : qa;
-    my_t0 = simd * q4 + (upper ? qa : 0);
+    const int base = q4 / (NW / 4), extra = q4 % (NW / 4);
+    my_n = base + (nth < extra ? 1 : 0);
+    my_t0 = simd * q4 + nth * base + (nth < extra ? nth : extra);
   } else {
     const int base = ntiles / nwaves, extra = ntiles % nwaves;
     my_n = base + (wave < extra ? 1 : 0);
     my_t0 = wave * base + (wave < extra ? wave : extra);
   }
-  const int my_np = upper ? n_rem : 0;  // k-quarter pieces of this wave
+  const int my_np = pieces ? n_rem : 0;  // k-quarter pieces of this wave
   T* qpart = reinterpret_cast<T*>(reinterpret_cast<char*>(red) + 8 * 4 * sizeof(double));
   int trow[NT], tcol[NT];
   // Where the FP32 form has an even number of row tiles, tiles are numbered
@@ -396,7 +397,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
 #pragma unroll
     for (int t = 0; t < NT; ++t)
       if (t < my_n) epilogue(acc[t], trow[t], tcol[t]);
-    if (upper && simd < n_rem) {
+    if (pieces && simd < n_rem) {
       // Remainder tile `simd`: the four quarters in order, then its epilogue.
       AccT sum = AccT{};
       const T* slot = qpart + (size_t)(simd * 4 * NACC) * 64 + lanee;
@@ -459,21 +460,28 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   __syncthreads();  // LDS is reused by the next tile
 }
 
-template <class TR, int NT>
+template <class TR, int NT, int NW>
 __device__ __forceinline__ void mte_tile(const MteJob& jb, const int tile, char* smem) {
   switch (jb.law) {
-    case kLawRefCpu: mte_tile_law<TR, kLawRefCpu, NT>(jb, tile, smem); break;
-    case kLawRefGpu: mte_tile_law<TR, kLawRefGpu, NT>(jb, tile, smem); break;
-    default: mte_tile_law<TR, kLawLognormal, NT>(jb, tile, smem); break;
+    case kLawRefCpu: mte_tile_law<TR, kLawRefCpu, NT, NW>(jb, tile, smem); break;
+    case kLawRefGpu: mte_tile_law<TR, kLawRefGpu, NT, NW>(jb, tile, smem); break;
+    default: mte_tile_law<TR, kLawLognormal, NT, NW>(jb, tile, smem); break;
   }
 }
 
-template <class TR, int NT>
-__global__ __launch_bounds__(kMteThreads) void mte_direct_kernel(
+// Two waves per SIMD: one workgroup of eight waves, or two of four (FP32
+// tiles of up to sixteen output tiles), which drift apart, so that one's
+// epilogue (VALU) runs beside the other's products (matrix cores): 26.0 ->
+// 23.7 ms for 3 species x 256 patches, 100 years, 100,000 paths.  Four waves
+// per SIMD with two tiles each instead (128 VGPRs) took 25.4 ms: twice the
+// splits per product, VALU issue 62% of the time.
+template <class TR, int NT, int NW>
+__global__ __launch_bounds__(NW * 64)
+__attribute__((amdgpu_waves_per_eu(2))) void mte_direct_kernel(
     const MteJob* __restrict__ jobs, const int2* __restrict__ work) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int2 w = work[blockIdx.x];
-  mte_tile<TR, NT>(jobs[w.x], w.y, smem);
+  mte_tile<TR, NT, NW>(jobs[w.x], w.y, smem);
 }
 
 // Persistent form.  The work items are split into nq queues, one per XCD,
@@ -482,8 +490,9 @@ __global__ __launch_bounds__(kMteThreads) void mte_direct_kernel(
 // XCDs round robin (workgroup b runs on XCD b % 8), so workgroup b first
 // drains queue b % nq and then takes what is left in the others.  Every
 // workgroup leaves each queue once its counter passes the queue length.
-template <class TR, int NT>
-__global__ __launch_bounds__(kMteThreads) void mte_persistent_kernel(
+template <class TR, int NT, int NW>
+__global__ __launch_bounds__(NW * 64)
+__attribute__((amdgpu_waves_per_eu(2))) void mte_persistent_kernel(
     const MteJob* __restrict__ jobs, const int2* __restrict__ work,
     const int* __restrict__ qbeg, int nq, int* __restrict__ counters) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -499,7 +508,7 @@ __global__ __launch_bounds__(kMteThreads) void mte_persistent_kernel(
       __syncthreads();
       if (w >= len) break;
       const int2 it = work[base + w];
-      mte_tile<TR, NT>(jobs[it.x], it.y, smem);
+      mte_tile<TR, NT, NW>(jobs[it.x], it.y, smem);
     }
   }
 }
@@ -528,69 +537,80 @@ __global__ void fill_i32_kernel(int* p, int v, int n) {
 
 namespace {
 
-// Kernel forms: FP64 and split-bf16 at their traits' tile bound; FP32 at 1, 2
-// or 4 tiles per wave.  direct selects mte_direct_kernel, else the persistent
-// kernel.
-template <class TR, int NT>
+// Kernel forms: FP64 and split-bf16 at their traits' tile bound and eight
+// waves; FP32 at 1, 2 or 4 tiles per wave and four or eight waves.  direct
+// selects mte_direct_kernel, else the persistent kernel.
+template <class TR, int NT, int NW>
 const void* mte_fn(bool direct) {
-  return direct ? reinterpret_cast<const void*>(&mte_direct_kernel<TR, NT>)
-                : reinterpret_cast<const void*>(&mte_persistent_kernel<TR, NT>);
+  return direct ? reinterpret_cast<const void*>(&mte_direct_kernel<TR, NT, NW>)
+                : reinterpret_cast<const void*>(&mte_persistent_kernel<TR, NT, NW>);
 }
 
-const void* mte_form(int prec, int tiles_per_wave, bool direct) {
+template <int NW>
+const void* mte_fn_f32(int tiles_per_wave, bool direct) {
+  if (tiles_per_wave <= 1) return mte_fn<TraitsX6, 1, NW>(direct);
+  if (tiles_per_wave <= 2) return mte_fn<TraitsX6, 2, NW>(direct);
+  return mte_fn<TraitsX6, TraitsX6::NT, NW>(direct);
+}
+
+const void* mte_form(int prec, int tiles_per_wave, int waves, bool direct) {
   switch (prec) {
-    case kPrecF64: return mte_fn<TraitsF64, TraitsF64::NT>(direct);
-    case kPrecB3: return mte_fn<TraitsB3, TraitsB3::NT>(direct);
+    case kPrecF64: return mte_fn<TraitsF64, TraitsF64::NT, 8>(direct);
+    case kPrecB3: return mte_fn<TraitsB3, TraitsB3::NT, 8>(direct);
     default:
-      if (tiles_per_wave <= 1) return mte_fn<TraitsX6, 1>(direct);
-      if (tiles_per_wave <= 2) return mte_fn<TraitsX6, 2>(direct);
-      return mte_fn<TraitsX6, TraitsX6::NT>(direct);
+      return waves == 4 ? mte_fn_f32<4>(tiles_per_wave, direct)
+                        : mte_fn_f32<8>(tiles_per_wave, direct);
   }
 }
 
 int mte_max_tiles_per_wave(int prec) {
-  return prec == kPrecF64 ? TraitsF64::NT : prec == kPrecB3 ? TraitsB3::NT : TraitsF32::NT;
+  return prec == kPrecF64 ? TraitsF64::NT : prec == kPrecB3 ? TraitsB3::NT : TraitsX6::NT;
+}
+
+bool mte_form_ok(int prec, int tiles_per_wave, int waves) {
+  return tiles_per_wave <= mte_max_tiles_per_wave(prec) &&
+         (waves == 8 || (waves == 4 && prec == kPrecF32));
 }
 
 }  // namespace
 
-int mte_tiles_per_wave(int prec, int BM, int Pp) {
-  const int tm = prec == kPrecF64 ? TraitsF64::TM : TraitsF32::TM;
-  const int tn = prec == kPrecF64 ? TraitsF64::TN : TraitsF32::TN;
-  const int nwaves = kMteThreads / 64;
-  return ((BM / tm) * (Pp / tn) + nwaves - 1) / nwaves;
+int mte_tiles_per_wave(int prec, int BM, int Pp, int waves) {
+  const int tm = prec == kPrecF64 ? TraitsF64::TM : TraitsX6::TM;
+  const int tn = prec == kPrecF64 ? TraitsF64::TN : TraitsX6::TN;
+  return ((BM / tm) * (Pp / tn) + waves - 1) / waves;
 }
 
 hipError_t mte_set_lds_limit(int prec, size_t bytes) {
   for (int tpw : {1, 2, 4})
-    for (bool direct : {true, false}) {
-      const hipError_t e = hipFuncSetAttribute(mte_form(prec, tpw, direct),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)bytes);
-      if (e != hipSuccess) return e;
-    }
+    for (int waves : {4, 8})
+      for (bool direct : {true, false}) {
+        const hipError_t e = hipFuncSetAttribute(mte_form(prec, tpw, waves, direct),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)bytes);
+        if (e != hipSuccess) return e;
+      }
   return hipSuccess;
 }
 
-hipError_t launch_mte_direct(int prec, int tiles_per_wave, const MteJob* jobs, const int2* work,
-                             int n_work, size_t lds, hipStream_t s) {
+hipError_t launch_mte_direct(int prec, int tiles_per_wave, int waves, const MteJob* jobs,
+                             const int2* work, int n_work, size_t lds, hipStream_t s) {
   if (n_work <= 0) return hipSuccess;
-  if (tiles_per_wave > mte_max_tiles_per_wave(prec)) return hipErrorInvalidValue;
+  if (!mte_form_ok(prec, tiles_per_wave, waves)) return hipErrorInvalidValue;
   void* args[] = {&jobs, &work};
-  const hipError_t e = hipLaunchKernel(mte_form(prec, tiles_per_wave, true), dim3(n_work),
-                                       dim3(kMteThreads), args, lds, s);
+  const hipError_t e = hipLaunchKernel(mte_form(prec, tiles_per_wave, waves, true), dim3(n_work),
+                                       dim3(waves * 64), args, lds, s);
   return e != hipSuccess ? e : hipGetLastError();
 }
 
-hipError_t launch_mte_persistent(int prec, int tiles_per_wave, const MteJob* jobs,
+hipError_t launch_mte_persistent(int prec, int tiles_per_wave, int waves, const MteJob* jobs,
                                  const int2* work, const int* qbeg, int nq,
                                  int* counters, int grid, size_t lds,
                                  hipStream_t s) {
   if (nq <= 0 || grid <= 0) return hipSuccess;
-  if (tiles_per_wave > mte_max_tiles_per_wave(prec)) return hipErrorInvalidValue;
+  if (!mte_form_ok(prec, tiles_per_wave, waves)) return hipErrorInvalidValue;
   void* args[] = {&jobs, &work, &qbeg, &nq, &counters};
-  const hipError_t e = hipLaunchKernel(mte_form(prec, tiles_per_wave, false), dim3(grid),
-                                       dim3(kMteThreads), args, lds, s);
+  const hipError_t e = hipLaunchKernel(mte_form(prec, tiles_per_wave, waves, false), dim3(grid),
+                                       dim3(waves * 64), args, lds, s);
   return e != hipSuccess ? e : hipGetLastError();
 }
 

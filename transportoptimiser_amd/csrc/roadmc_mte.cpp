@@ -226,12 +226,25 @@ struct JobSet {
   std::vector<MteJob> jobs;
   std::vector<int> road_of, species_of;
   std::vector<int64_t> mpack_off, cols_off, part_off, out_off, endpop_off;
+  std::vector<int> waves;  // of each job's workgroups
   std::vector<int2> work;
-  std::vector<int> qbeg;  // per-XCD queue boundaries into work (persistent)
   size_t mpack_elems = 0, cols_elems = 0, part_elems = 0, out_elems = 0,
          endpop_elems = 0;
-  size_t lds = 0;
-  int tpw = 1;  // most output tiles per wave over the jobs
+  // The launches: jobs by the waves of their workgroups, the larger first.
+  struct Launch {
+    int waves = 8;
+    size_t lds = 0;
+    int tpw = 1;                  // most output tiles per wave over the jobs
+    int work0 = 0, n_work = 0;    // its items of work
+    std::vector<int> qbeg;        // per-XCD queue boundaries, from work0 (persistent)
+    int grid = 0;                 // persistent workgroups
+  };
+  std::vector<Launch> launches;
+  size_t lds_max() const {
+    size_t m = 0;
+    for (const Launch& l : launches) m = std::max(m, l.lds);
+    return m;
+  }
 };
 
 void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roads,
@@ -275,46 +288,70 @@ void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roa
       if (want_end_pops) js.endpop_elems += (size_t)jb.N;
       // Remainder tiles (ntiles % 4) would leave one SIMD with more work
       // than the others; split them into k-quarters when LDS has room for
-      // the partial products (FP32 kernel, at least 8 k-groups).
+      // the partial products (FP32 and split-bf16 kernels, at least 8
+      // k-groups).
       const int ntiles = (jb.BM / roadmc::kMteRowsF32) * (jb.Pp / 32);
       const int rem = ntiles % 4;
-      jb.split = 0;
-      if (!js.fp64 && rem && ctx->tiles[tile_slot(js.prec)][bucket_of(jb.Pp)].split &&
-          (jb.Pk >> 3) >= 8 &&
-          roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem) <= kLdsPerCu)
-        jb.split = 1;
-      js.lds = std::max(js.lds, roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp,
-                                                      jb.split ? rem : 0));
-      js.tpw = std::max(js.tpw, roadmc::mte_tiles_per_wave(js.prec, jb.BM, jb.Pp));
+      const bool may_split = !js.fp64 && rem &&
+                             ctx->tiles[tile_slot(js.prec)][bucket_of(jb.Pp)].split &&
+                             (jb.Pk >> 3) >= 8;
+      const size_t lds0 = roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, 0);
+      const size_t lds_rem = roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem);
+      // FP32 tiles of at most 16 output tiles run as four-wave workgroups,
+      // two of them on a CU (see mte_kernels.hip); larger ones, and those
+      // whose LDS leaves no room for a second, as eight-wave workgroups.
+      int waves = 8;
+      jb.split = may_split && lds_rem <= kLdsPerCu;
+      if (js.prec == roadmc::kPrecF32 && ntiles <= roadmc::kMteTilesFourWaves &&
+          2 * lds0 <= kLdsPerCu) {
+        waves = 4;
+        jb.split = may_split && 2 * lds_rem <= kLdsPerCu;
+      }
       js.jobs.push_back(jb);
+      js.waves.push_back(waves);
       js.road_of.push_back(r);
       js.species_of.push_back(s);
     }
   }
   // Jobs in decreasing cost (cost ~ n_tiles * BM * Pp^2 * T), assigned to
-  // the per-XCD queues by longest-processing-time-first; each queue lists
-  // its jobs' tiles contiguously.
-  std::vector<int> order(js.jobs.size());
-  for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
+  // the per-XCD queues of their launch by longest-processing-time-first; each
+  // queue lists its jobs' tiles contiguously.
   auto cost = [&](int j) {
     const MteJob& x = js.jobs[j];
     return (double)x.n_tiles * x.BM * x.Pp * x.Pp * x.T;
   };
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int a, int b) { return cost(a) > cost(b); });
   const int nq = roadmc::kMteQueues;
-  std::vector<std::vector<int>> queues(nq);
-  std::vector<double> load(nq, 0.0);
-  for (int j : order) {
-    const int q = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    queues[q].push_back(j);
-    load[q] += cost(j);
-  }
-  js.qbeg.assign(1, 0);
-  for (int q = 0; q < nq; ++q) {
-    for (int j : queues[q])
-      for (int t = 0; t < js.jobs[j].n_tiles; ++t) js.work.push_back(make_int2(j, t));
-    js.qbeg.push_back((int)js.work.size());
+  for (int waves : {8, 4}) {
+    JobSet::Launch l;
+    l.waves = waves;
+    std::vector<int> order;
+    for (size_t j = 0; j < js.jobs.size(); ++j) {
+      if (js.waves[j] != waves) continue;
+      order.push_back((int)j);
+      const MteJob& jb = js.jobs[j];
+      const int rem = jb.split ? (jb.BM / roadmc::kMteRowsF32) * (jb.Pp / 32) % 4 : 0;
+      l.lds = std::max(l.lds, roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem));
+      l.tpw = std::max(l.tpw, roadmc::mte_tiles_per_wave(js.prec, jb.BM, jb.Pp, waves));
+    }
+    if (order.empty()) continue;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int a, int b) { return cost(a) > cost(b); });
+    std::vector<std::vector<int>> queues(nq);
+    std::vector<double> load(nq, 0.0);
+    for (int j : order) {
+      const int q = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      queues[q].push_back(j);
+      load[q] += cost(j);
+    }
+    l.work0 = (int)js.work.size();
+    l.qbeg.assign(1, 0);
+    for (int q = 0; q < nq; ++q) {
+      for (int j : queues[q])
+        for (int t = 0; t < js.jobs[j].n_tiles; ++t) js.work.push_back(make_int2(j, t));
+      l.qbeg.push_back((int)js.work.size() - l.work0);
+    }
+    l.n_work = (int)js.work.size() - l.work0;
+    js.launches.push_back(l);
   }
 }
 
@@ -398,9 +435,13 @@ int upload_jobs(roadmc_ctx* ctx, const roadmc_mte_problem* roads, JobSet& js,
                               hipMemcpyHostToDevice, s));
   RMC_HIP(ctx, hipMemcpyAsync(b.off.ptr, js.out_off.data(),
                               js.out_off.size() * sizeof(int64_t), hipMemcpyHostToDevice, s));
-  // Queue boundaries live after the 16 queue counters in the counter buffer.
-  RMC_HIP(ctx, hipMemcpyAsync(static_cast<int*>(b.counter.ptr) + 16, js.qbeg.data(),
-                              js.qbeg.size() * sizeof(int), hipMemcpyHostToDevice, s));
+  // The counter buffer: 8 queue counters of each launch, then from 16 the
+  // queue boundaries, 16 entries a launch.
+  for (size_t l = 0; l < js.launches.size(); ++l)
+    RMC_HIP(ctx, hipMemcpyAsync(static_cast<int*>(b.counter.ptr) + 16 + 16 * l,
+                                js.launches[l].qbeg.data(),
+                                js.launches[l].qbeg.size() * sizeof(int), hipMemcpyHostToDevice,
+                                s));
   // Species given by a road: build trans and surv on the device and pack
   // them into their job's slot (after the upload above).  Every road's
   // inputs go up in one copy; the builds then run one after the other in
@@ -747,10 +788,12 @@ extern "C" int roadmc_mte_run(roadmc_ctx* ctx, const roadmc_mte_problem* problem
   rc = js.fp64 ? upload_jobs<double>(ctx, problem, js, b, false)
                : upload_jobs<float>(ctx, problem, js, b, false);
   if (rc) return rc;
-  if ((rc = ensure_lds_limit(ctx, js.prec, js.lds))) return rc;
-  RMC_HIP(ctx, roadmc::launch_mte_direct(js.prec, js.tpw, static_cast<MteJob*>(b.jobs.ptr),
-                                         static_cast<int2*>(b.work.ptr), (int)js.work.size(),
-                                         js.lds, ctx->stream));
+  if ((rc = ensure_lds_limit(ctx, js.prec, js.lds_max()))) return rc;
+  for (const JobSet::Launch& l : js.launches)
+    RMC_HIP(ctx, roadmc::launch_mte_direct(js.prec, l.tpw, l.waves,
+                                           static_cast<MteJob*>(b.jobs.ptr),
+                                           static_cast<int2*>(b.work.ptr) + l.work0, l.n_work,
+                                           l.lds, ctx->stream));
   RMC_HIP(ctx, roadmc::launch_mte_reduce(static_cast<MteJob*>(b.jobs.ptr), (int)js.jobs.size(),
                                          static_cast<double*>(b.out.ptr),
                                          static_cast<int64_t*>(b.off.ptr), ctx->stream));
@@ -768,7 +811,6 @@ struct roadmc_batch {
   std::vector<std::vector<roadmc_species>> species;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  int grid = 0;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
   size_t timed_from = 0;
 };
@@ -780,13 +822,27 @@ int capture_batch_graph(roadmc_batch* bt) {
   hipStream_t s = ctx->stream;
   JobSet& js = bt->js;
   JobBuffers& b = bt->bufs;
+  if (js.launches.size() > 1 && !ctx->batch_side) {
+    RMC_HIP(ctx, hipEventCreateWithFlags(&ctx->batch_fork, hipEventDisableTiming));
+    RMC_HIP(ctx, hipEventCreateWithFlags(&ctx->batch_join, hipEventDisableTiming));
+    RMC_HIP(ctx, hipStreamCreateWithFlags(&ctx->batch_side, hipStreamNonBlocking));
+  }
   RMC_HIP(ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   hipError_t e = roadmc::launch_fill_i32(static_cast<int*>(b.counter.ptr), 0, 16, s);
-  if (e == hipSuccess)
+  // Two launches run side by side: the small tiles fill the CUs that the
+  // large tiles' last round leaves.
+  const bool fork = js.launches.size() > 1;
+  if (e == hipSuccess && fork) e = hipEventRecord(ctx->batch_fork, s);
+  if (e == hipSuccess && fork) e = hipStreamWaitEvent(ctx->batch_side, ctx->batch_fork, 0);
+  for (size_t l = 0; l < js.launches.size() && e == hipSuccess; ++l)
     e = roadmc::launch_mte_persistent(
-        js.prec, js.tpw, static_cast<MteJob*>(b.jobs.ptr), static_cast<int2*>(b.work.ptr),
-        static_cast<int*>(b.counter.ptr) + 16, (int)js.qbeg.size() - 1,
-        static_cast<int*>(b.counter.ptr), bt->grid, js.lds, s);
+        js.prec, js.launches[l].tpw, js.launches[l].waves, static_cast<MteJob*>(b.jobs.ptr),
+        static_cast<int2*>(b.work.ptr) + js.launches[l].work0,
+        static_cast<int*>(b.counter.ptr) + 16 + 16 * l, (int)js.launches[l].qbeg.size() - 1,
+        static_cast<int*>(b.counter.ptr) + 8 * l, js.launches[l].grid, js.launches[l].lds,
+        l ? ctx->batch_side : s);
+  if (e == hipSuccess && fork) e = hipEventRecord(ctx->batch_join, ctx->batch_side);
+  if (e == hipSuccess && fork) e = hipStreamWaitEvent(s, ctx->batch_join, 0);
   if (e == hipSuccess)
     e = roadmc::launch_mte_reduce(static_cast<MteJob*>(b.jobs.ptr), (int)js.jobs.size(),
                                   static_cast<double*>(b.out.ptr),
@@ -829,18 +885,20 @@ extern "C" int roadmc_batch_prepare(roadmc_ctx* ctx, const roadmc_mte_problem* r
   plan_jobs(ctx, roads, n_roads, true, bt->js);
   int rc = bt->js.fp64 ? upload_jobs<double>(ctx, roads, bt->js, bt->bufs, true)
                        : upload_jobs<float>(ctx, roads, bt->js, bt->bufs, true);
-  if (!rc) rc = ensure_lds_limit(ctx, bt->js.prec, bt->js.lds);
+  if (!rc) rc = ensure_lds_limit(ctx, bt->js.prec, bt->js.lds_max());
   if (!rc) {
     // One workgroup per CU fits the LDS of the largest tile; small tiles
-    // leave room for a second one, unless a bucket of the batch asks for one.
-    int want = 2;
-    if (!bt->js.fp64)
-      for (const MteJob& jb : bt->js.jobs) {
-        const int pc = ctx->tiles[tile_slot(bt->js.prec)][bucket_of(jb.Pp)].per_cu;
+    // leave room for a second one, unless a bucket of the launch asks for one.
+    for (JobSet::Launch& l : bt->js.launches) {
+      int want = 2;
+      for (size_t j = 0; j < bt->js.jobs.size() && !bt->js.fp64; ++j) {
+        if (bt->js.waves[j] != l.waves) continue;
+        const int pc =
+            ctx->tiles[tile_slot(bt->js.prec)][bucket_of(bt->js.jobs[j].Pp)].per_cu;
         want = std::min(want, pc == 0 ? 2 : pc);
       }
-    const int per_cu = (want == 2 && bt->js.lds * 2 <= kLdsPerCu) ? 2 : 1;
-    bt->grid = ctx->n_cu * per_cu;
+      l.grid = ctx->n_cu * ((want == 2 && l.lds * 2 <= kLdsPerCu) ? 2 : 1);
+    }
     bt->roads.assign(roads, roads + n_roads);
     rc = capture_batch_graph(bt);
   }
@@ -1465,13 +1523,17 @@ extern "C" int roadmc_mte_adjoint_fwd(roadmc_ctx* ctx, const roadmc_mte_problem*
   std::vector<int2> work(jb.n_tiles);
   for (int t = 0; t < jb.n_tiles; ++t) work[t] = make_int2(0, t);
   const int64_t off0 = 0;
-  const size_t lds = roadmc::mte_lds_bytes(adj->fp64 ? roadmc::kPrecF64 : roadmc::kPrecF32, jb.BM, jb.Pp, 0);
+  const int prec = adj->fp64 ? roadmc::kPrecF64 : roadmc::kPrecF32;
+  const int waves =
+      !adj->fp64 && (jb.BM / roadmc::kMteRowsF32) * (jb.Pp / 32) <= roadmc::kMteTilesFourWaves ? 4
+                                                                                               : 8;
+  const size_t lds = roadmc::mte_lds_bytes(prec, jb.BM, jb.Pp, 0);
   hipStream_t s = ctx->stream;
   auto fail = [&](int code) {
     roadmc_adjoint_destroy(adj);
     return code;
   };
-  if ((rc = ensure_lds_limit(ctx, adj->fp64 ? roadmc::kPrecF64 : roadmc::kPrecF32, lds))) return fail(rc);
+  if ((rc = ensure_lds_limit(ctx, prec, lds))) return fail(rc);
   hipError_t e = hipMemcpyAsync(adj->bufs.jobs.ptr, &jb, sizeof(MteJob), hipMemcpyHostToDevice, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(adj->bufs.work.ptr, work.data(), work.size() * sizeof(int2),
@@ -1479,11 +1541,8 @@ extern "C" int roadmc_mte_adjoint_fwd(roadmc_ctx* ctx, const roadmc_mte_problem*
   if (e == hipSuccess)
     e = hipMemcpyAsync(adj->bufs.off.ptr, &off0, sizeof(off0), hipMemcpyHostToDevice, s);
   if (e == hipSuccess)
-    e = roadmc::launch_mte_direct(adj->fp64 ? roadmc::kPrecF64 : roadmc::kPrecF32,
-                                  roadmc::mte_tiles_per_wave(adj->fp64 ? roadmc::kPrecF64
-                                                                       : roadmc::kPrecF32,
-                                                             jb.BM, jb.Pp),
-                                  static_cast<MteJob*>(adj->bufs.jobs.ptr),
+    e = roadmc::launch_mte_direct(prec, roadmc::mte_tiles_per_wave(prec, jb.BM, jb.Pp, waves),
+                                  waves, static_cast<MteJob*>(adj->bufs.jobs.ptr),
                                   static_cast<int2*>(adj->bufs.work.ptr), jb.n_tiles, lds, s);
   if (e == hipSuccess)
     e = roadmc::launch_mte_reduce(static_cast<MteJob*>(adj->bufs.jobs.ptr), 1,
