@@ -163,10 +163,12 @@ void roadmc_batch_destroy(roadmc_batch* batch);
 /* Tile settings of the MTE launches, per precision (ROADMC_PREC_FP32 or
  * ROADMC_PREC_BF16X3; FP64 tiles follow LDS) and patch-count bucket
  * (P <= 128, 256, 512, 1024): rows of paths per workgroup (a power of two in
- * [32, 256], rows x P <= 32768); split 1 lets remainder tiles (the tiles left
- * after an even share per SIMD) be computed as four k-quarters, 0 not;
+ * [32, 256], rows x P <= 32768); split 1 lets BF16X3's remainder tiles (the tiles
+ * left after an even share per SIMD) be computed as four k-quarters, 0 not
+ * (the FP32 kernels never do);
  * per_cu 1 or 2 workgroups per CU of the persistent launch (0: two when LDS
  * allows; a batch takes the smallest of its buckets' values).
+ * An FP32 launch with fewer workgroups than CUs takes fewer rows.
  * Rows and per_cu never change results (each path's products and draws are
  * the same in any tile); a split changes the k-summation order of the split
  * tiles' paths, so their end totals move within FP32 rounding.

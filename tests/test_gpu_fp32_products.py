@@ -47,3 +47,22 @@ def test_one_year_product_within_the_fp32_bound(ctx, N):
             err = np.abs(out.patch_mean[0] - ref) / ref
             assert err.max() <= bound, (P, err.max(), bound)
             np.testing.assert_allclose(out.end_pops[:, 0], ref.sum(), rtol=bound)
+
+
+def test_small_launch_takes_fewer_rows_with_the_same_bits(ctx):
+    # Alone each road leaves CUs idle and takes 32-row tiles, the smallest with
+    # several waves to a tile; with the large one in the batch they take the
+    # tile table's rows.
+    roads = []
+    for i, (P, N) in enumerate([(20, 700), (33, 1000), (100, 1500), (256, 3000), (400, 900)]):
+        sp = ls.make_species(np.random.default_rng(70 + i), P)
+        roads.append(ls.RoadProblem([sp], n_years=4, n_paths=N, seed=2, road_id=i))
+    big = ls.RoadProblem([ls.make_species(np.random.default_rng(80), 64)], n_years=1,
+                         n_paths=60000, seed=2, road_id=9)
+    print("small roads alone, then in a batch", flush=True)
+    alone = [ctx.simulate_mte(r) for r in roads]
+    batch = ctx.simulate_mte_batch(roads + [big], end_pops=True)
+    for a, b in zip(alone, batch):
+        for x, y in ((a.end_pops, b.end_pops), (a.end_mean, b.end_mean), (a.end_sd, b.end_sd),
+                     (a.patch_mean[0], b.patch_mean[0]), (a.mte_prob, b.mte_prob)):
+            np.testing.assert_array_equal(x, y)

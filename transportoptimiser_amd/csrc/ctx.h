@@ -29,13 +29,14 @@ struct roadmc_ctx {
   size_t lds_limit_f32 = 0, lds_limit_f64 = 0, lds_limit_b3 = 0;
   // Tile settings of the MTE launches per precision (0: FP32, 1: split bf16)
   // and patch-count bucket (P <= 128, 256, 512, 1024): rows of paths per
-  // workgroup; whether remainder tiles may be split over k (1) or not (0);
+  // workgroup; whether remainder tiles may be split over k (1, split bf16
+  // only) or not (0);
   // workgroups per CU of the persistent launch (0: as many as LDS allows,
   // else 1 or 2).  Set by roadmc_set_tile or roadmc_autotune_ex.
   struct TileSetting {
     int rows, split, per_cu;
   };
-  TileSetting tiles[2][4] = {{{128, 1, 0}, {64, 1, 0}, {64, 1, 0}, {32, 1, 0}},
+  TileSetting tiles[2][4] = {{{128, 0, 0}, {64, 0, 0}, {64, 0, 0}, {32, 0, 0}},
                              {{256, 1, 0}, {128, 1, 0}, {64, 1, 0}, {32, 1, 0}}};
   rmc_job_buffers mte_bufs;
   struct {

@@ -21,13 +21,14 @@ struct MteJob {
   double* end_pops;    // [N] per-path end totals, or nullptr
   void* ckpt;          // adjoint checkpoints [T/ckpt_every][N][Pp], or nullptr
   int32_t ckpt_every;
-  double* partial;     // [n_tiles][3 + Pp]: count, sum, sum of squares,
-                       // per-patch sums of one tile
+  double* partial;     // [n_part][3 + Pp]: count, sum, sum of squares,
+                       // per-patch sums of one block of paths (32 in the
+                       // FP32 kernels, else a tile)
   double params[8];    // packed species parameters (SimulateGPU.cu:3690-3714)
   double sigma;        // LOGNORMAL year-noise SD
   double dt;           // time step
   double thr_total;    // threshold_ratio * initial total
-  int32_t P, Pp, N, T, BM, law, endpoint, n_tiles;
+  int32_t P, Pp, N, T, BM, law, endpoint, n_tiles, n_part;
   int32_t Pk;          // contraction extent: P rounded up to 16 (<= Pp); Pp
                        // in the split-bf16 form (an even count of 16-k chunks)
   int32_t split;       // split the ntiles % 4 remainder tiles into k-quarters

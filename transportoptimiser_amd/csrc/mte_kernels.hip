@@ -130,6 +130,19 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
     my_n = base + (wave < extra ? 1 : 0);
     my_t0 = wave * base + (wave < extra ? wave : extra);
   }
+  // Fewer tiles than waves (the smallest roads): `parts` waves form one tile's
+  // product alike and each applies the epilogue to its share of the path
+  // quads, the year's longest chain.
+  int parts = 1, share = 0;
+  if constexpr (kX6 && NT == 1) {
+    if (ntiles < nwaves) {
+      parts = min(4, nwaves / ntiles);
+      parts = parts == 3 ? 2 : parts;
+      share = wave / ntiles;
+      my_n = share < parts ? 1 : 0;
+      my_t0 = wave - share * ntiles;
+    }
+  }
   const int my_np = pieces ? n_rem : 0;  // k-quarter pieces of this wave
   T* qpart = reinterpret_cast<T*>(reinterpret_cast<char*>(red) + 8 * 4 * sizeof(double));
   int trow[NT], tcol[NT];
@@ -219,20 +232,8 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       }
 #undef RMC_YP3
     } else if constexpr (kX6) {
-      // The same schedule: k-quarter pieces first, then the whole tiles in
-      // blocks of 2 x 2, 2 x 1, 1 x 2 or single tiles.
+      // Blocks of 2 x 2, 2 x 1, 1 x 2 or single tiles.
       const float* const Al = A + arow * LDAy + akoff;
-      for (int i = 0; i < my_np; ++i) {
-        int tr, tc;
-        tile_pos(4 * q4 + i, tr, tc);
-        AccT pacc;
-        const uint32_t bo = b6_voff(nch, tc, lane);
-        product_x6<1, 1>(&pacc, Bm, Al + tr * TM * LDAy, 0, &bo, (simd * nch) >> 2,
-                         ((simd + 1) * nch) >> 2);
-        T* slot = qpart + (size_t)((i * 4 + simd) * NACC) * 64 + lane;
-#pragma unroll
-        for (int r = 0; r < NACC; ++r) slot[r * 64] = pacc[r];
-      }
       // No value of last year's accumulators lives across the products.
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[t] = AccT{};
@@ -362,6 +363,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       const T ga = (T)1 + rr * rscale, gb = rr * rscale * Ki;
 #pragma unroll
       for (int r4 = 0; r4 < NACC; r4 += 4) {
+        if (kX6 && NT == 1 && r4 * parts / NACC != share) continue;
         T z[4];
         if constexpr (TR::kQuadItems) {
           const int row0 = tr * TM + TR::acc_row(lanee, r4);
@@ -423,6 +425,39 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       return (double)A[r * LDA + c];
     }
   };
+  if constexpr (kX6) {
+    // One partial per block of 32 rows, so that the sums over the blocks do
+    // not depend on the tile's rows.  nthreads >= BM: a row to a thread, a
+    // block of rows to a half-wave.
+    RMC_GLOBAL double* const part0 = gmem(jb.partial) + (size_t)(p0 >> 5) * (3 + Pp);
+    if (tid < BM) {
+      const int path = p0 + tid;
+      double v[3] = {0.0, 0.0, 0.0};
+      if (path < jb.N) {
+        double tot = 0.0;
+        for (int c = 0; c < Pp; ++c) tot += state_at(tid, c);
+        if (jb.end_pops) gmem(jb.end_pops)[path] = tot;
+        v[0] = tot >= jb.thr_total ? 1.0 : 0.0;
+        v[1] = tot;
+        v[2] = tot * tot;
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) v[i] += __shfl_xor(v[i], off, 64);
+        if ((tid & 31) == 0 && path < jb.N) part0[(size_t)(tid >> 5) * (3 + Pp) + i] = v[i];
+      }
+    }
+    for (int i = tid; i < (BM >> 5) * Pp; i += nthreads) {
+      const int rb = i / Pp, c = i - rb * Pp;
+      const int n = min(32, jb.N - p0 - 32 * rb);
+      double s = 0.0;
+      for (int r = 0; r < n; ++r) s += state_at(32 * rb + r, c);
+      if (n > 0) part0[(size_t)rb * (3 + Pp) + 3 + c] = s;
+    }
+    __syncthreads();  // LDS is reused by the next tile
+    return;
+  }
   double cnt = 0.0, sum = 0.0, sq = 0.0;
   for (int r = tid; r < BM; r += nthreads) {
     const int path = p0 + r;
@@ -513,20 +548,36 @@ __attribute__((amdgpu_waves_per_eu(2))) void mte_persistent_kernel(
   }
 }
 
-// Sums the tile partials of each job in a fixed order (deterministic).
-__global__ void mte_reduce_kernel(const MteJob* __restrict__ jobs,
-                                  double* __restrict__ out,
-                                  const int64_t* __restrict__ out_off) {
+// Sums the partials of each job in a fixed order (deterministic): 32 columns
+// a workgroup, its 16 rows of threads each adding a contiguous sixteenth of
+// the partials, then those in order.  One thread per column over all partials
+// waited on memory: 53 us for 1,563 partials of 259 columns.
+constexpr int kReduceCols = 32, kReduceParts = 16;
+__global__ __launch_bounds__(kReduceCols* kReduceParts) void mte_reduce_kernel(
+    const MteJob* __restrict__ jobs, double* __restrict__ out,
+    const int64_t* __restrict__ out_off) {
+  __shared__ double sums[kReduceParts][kReduceCols];
   const MteJob& jb = jobs[blockIdx.x];
-  const int W = 3 + jb.Pp;
+  const int W = 3 + jb.Pp, x = threadIdx.x % kReduceCols, y = threadIdx.x / kReduceCols;
+  const RMC_GLOBAL double* part = gmem(jb.partial);
   double* o = out + out_off[blockIdx.x];
-  for (int e = threadIdx.x; e < W; e += blockDim.x) {
+  for (int e0 = blockIdx.y * kReduceCols; e0 < W; e0 += gridDim.y * kReduceCols) {
+    const int e = e0 + x;
+    const int t1 = (int)((int64_t)jb.n_part * (y + 1) / kReduceParts);
     double s = 0.0;
-    // Unrolled so that eight tiles' loads are in flight; the sum keeps its
-    // tile order.
+    if (e < W) {
+      // Unrolled so that eight partials' loads are in flight.
 #pragma unroll 8
-    for (int t = 0; t < jb.n_tiles; ++t) s += gmem(jb.partial)[(size_t)t * W + e];
-    o[e] = s;
+      for (int t = (int)((int64_t)jb.n_part * y / kReduceParts); t < t1; ++t)
+        s += part[(size_t)t * W + e];
+    }
+    sums[y][x] = s;
+    __syncthreads();
+    if (y == 0 && e < W) {
+      for (int i = 1; i < kReduceParts; ++i) s += sums[i][x];
+      o[e] = s;
+    }
+    __syncthreads();
   }
 }
 
@@ -678,8 +729,8 @@ hipError_t launch_mte_split_b3(float* m, size_t n_floats, hipStream_t s) {
 hipError_t launch_mte_reduce(const MteJob* jobs, int n_jobs, double* out,
                              const int64_t* out_off, hipStream_t s) {
   if (n_jobs <= 0) return hipSuccess;
-  hipLaunchKernelGGL(mte_reduce_kernel, dim3(n_jobs), dim3(256), 0, s, jobs,
-                     out, out_off);
+  hipLaunchKernelGGL(mte_reduce_kernel, dim3(n_jobs, 16), dim3(kReduceCols * kReduceParts), 0, s,
+                     jobs, out, out_off);
   return hipGetLastError();
 }
 

@@ -251,6 +251,28 @@ void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roa
                bool want_end_pops, JobSet& js) {
   js.prec = roads[0].precision;
   js.fp64 = js.prec == ROADMC_PREC_FP64;
+  const bool f32 = js.prec == roadmc::kPrecF32;
+  // Rows of paths per workgroup: the tile table's; in FP32, where a path's
+  // result does not depend on them, halved (down to 32) while the launch has
+  // fewer workgroups than the card has CUs: 256 patches and 5,000 paths
+  // 1.27 -> 0.84 ms, 100 patches and 2,000 paths 0.78 -> 0.54 ms.
+  int shrink = 1;
+  auto rows_of = [&](const roadmc_mte_problem& pr, int Pp) {
+    const int granule = js.fp64 ? roadmc::kMteRowsF64 : roadmc::kMteRowsF32;
+    return std::max(granule,
+                    rows_for(ctx, js.prec, Pp, pr.n_paths) / shrink / granule * granule);
+  };
+  auto workgroups = [&]() {
+    int64_t n = 0;
+    for (int r = 0; r < n_roads; ++r)
+      for (int s = 0; s < roads[r].n_species; ++s) {
+        const int bm = rows_of(roads[r], round_up(roads[r].species[s].n_patches, 32));
+        n += (roads[r].n_paths + bm - 1) / bm;
+      }
+    return n;
+  };
+  while (f32 && shrink < 8 && workgroups() < ctx->n_cu) shrink *= 2;
+  const bool fills = workgroups() > ctx->n_cu;
   for (int r = 0; r < n_roads; ++r) {
     const roadmc_mte_problem& pr = roads[r];
     for (int s = 0; s < pr.n_species; ++s) {
@@ -262,10 +284,12 @@ void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roa
       jb.Pk = js.prec == roadmc::kPrecB3 ? jb.Pp : round_up(jb.P, 16);
       jb.N = (int32_t)pr.n_paths;
       jb.T = pr.n_years;
-      jb.BM = rows_for(ctx, js.prec, jb.Pp, pr.n_paths);
+      jb.BM = rows_of(pr, jb.Pp);
       jb.law = pr.growth_law;
       jb.endpoint = pr.endpoint;
       jb.n_tiles = (int)((pr.n_paths + jb.BM - 1) / jb.BM);
+      jb.n_part = f32 ? (int)((pr.n_paths + roadmc::kMteRowsF32 - 1) / roadmc::kMteRowsF32)
+                      : jb.n_tiles;
       for (int i = 0; i < 8; ++i) jb.params[i] = sp.params[i];
       jb.sigma = sp.noise_sd;
       jb.dt = pr.time_step;
@@ -283,30 +307,28 @@ void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roa
       js.endpop_off.push_back(want_end_pops ? (int64_t)js.endpop_elems : -1);
       js.mpack_elems += (size_t)jb.Pp * jb.Pk;
       js.cols_elems += 4 * (size_t)jb.Pp;
-      js.part_elems += (size_t)jb.n_tiles * (3 + jb.Pp);
+      js.part_elems += (size_t)jb.n_part * (3 + jb.Pp);
       js.out_elems += 3 + (size_t)jb.Pp;
       if (want_end_pops) js.endpop_elems += (size_t)jb.N;
-      // Remainder tiles (ntiles % 4) would leave one SIMD with more work
-      // than the others; split them into k-quarters when LDS has room for
-      // the partial products (FP32 and split-bf16 kernels, at least 8
-      // k-groups).
+      // Split bf16: remainder tiles (ntiles % 4) would leave one SIMD with
+      // more work than the others; split them into k-quarters when LDS has
+      // room for the partial products (at least 8 k-groups).  The FP32 kernels
+      // never split: without it they are as fast or faster at every P (10.3
+      // against 11.7 ms at 480 patches, the same on a generation), and a path's
+      // result does not depend on the tile's rows or waves.
       const int ntiles = (jb.BM / roadmc::kMteRowsF32) * (jb.Pp / 32);
       const int rem = ntiles % 4;
-      const bool may_split = !js.fp64 && rem &&
-                             ctx->tiles[tile_slot(js.prec)][bucket_of(jb.Pp)].split &&
-                             (jb.Pk >> 3) >= 8;
-      const size_t lds0 = roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, 0);
-      const size_t lds_rem = roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem);
+      jb.split = js.prec == roadmc::kPrecB3 && rem &&
+                 ctx->tiles[tile_slot(js.prec)][bucket_of(jb.Pp)].split && (jb.Pk >> 3) >= 8 &&
+                 roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem) <= kLdsPerCu;
       // FP32 tiles of at most 16 output tiles run as four-wave workgroups,
-      // two of them on a CU (see mte_kernels.hip); larger ones, and those
-      // whose LDS leaves no room for a second, as eight-wave workgroups.
-      int waves = 8;
-      jb.split = may_split && lds_rem <= kLdsPerCu;
-      if (js.prec == roadmc::kPrecF32 && ntiles <= roadmc::kMteTilesFourWaves &&
-          2 * lds0 <= kLdsPerCu) {
-        waves = 4;
-        jb.split = may_split && 2 * lds_rem <= kLdsPerCu;
-      }
+      // two of them on a CU (see mte_kernels.hip); larger ones, those whose LDS
+      // leaves no room for a second and those of a launch without a second
+      // workgroup for some CU as eight-wave workgroups.
+      const int waves = f32 && fills && ntiles <= roadmc::kMteTilesFourWaves &&
+                                2 * roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, 0) <= kLdsPerCu
+                            ? 4
+                            : 8;
       js.jobs.push_back(jb);
       js.waves.push_back(waves);
       js.road_of.push_back(r);
@@ -623,7 +645,7 @@ int mte_run_wide(roadmc_ctx* ctx, const roadmc_mte_problem* pr, roadmc_mte_resul
     jb.BM = kB;
     jb.law = pr->growth_law;
     jb.endpoint = pr->endpoint;
-    jb.n_tiles = (int)((N + kB - 1) / kB);
+    jb.n_tiles = jb.n_part = (int)((N + kB - 1) / kB);
     for (int i = 0; i < 8; ++i) jb.params[i] = sp.params[i];
     jb.sigma = sp.noise_sd;
     jb.dt = pr->time_step;
@@ -1111,7 +1133,7 @@ extern "C" int roadmc_autotune_ex(roadmc_ctx* ctx, int32_t precision, int32_t n_
       // Two workgroups per CU only where the largest road's tile (with a
       // split's partial products) leaves room for a second.
       const size_t lds_max = roadmc::mte_lds_bytes(precision, rows, P, 3);
-      for (int split = 0; split <= 1; ++split) {
+      for (int split = 0; split <= (precision == ROADMC_PREC_BF16X3 ? 1 : 0); ++split) {
         const size_t lds = split ? lds_max : roadmc::mte_lds_bytes(precision, rows, P, 0);
         for (int per_cu = 1; per_cu <= (lds * 2 <= kLdsPerCu ? 2 : 1); ++per_cu) {
           ctx->tiles[slot][b] = {rows, split, per_cu};
@@ -1482,7 +1504,7 @@ extern "C" int roadmc_mte_adjoint_fwd(roadmc_ctx* ctx, const roadmc_mte_problem*
   jb.BM = adj->fp64 ? rows_for(ctx, ROADMC_PREC_FP64, jb.Pp, pr->n_paths) : roadmc::kMteRowsF32;
   jb.law = ROADMC_LAW_LOGNORMAL;
   jb.endpoint = ROADMC_END_POST_GROWTH;
-  jb.n_tiles = (int)((pr->n_paths + jb.BM - 1) / jb.BM);
+  jb.n_tiles = jb.n_part = (int)((pr->n_paths + jb.BM - 1) / jb.BM);
   for (int i = 0; i < 8; ++i) jb.params[i] = sp.params[i];
   jb.sigma = sp.noise_sd;
   jb.dt = pr->time_step;
