@@ -9,6 +9,8 @@ namespace roadmc {
 constexpr int kMlpMaxIn = 16;
 constexpr int kMlpMaxOut = 4;
 constexpr int kMlpMaxMembers = 8;
+constexpr int kMlpChunk = 32;  // samples per gradient or prediction block
+inline int mlp_chunks(int n) { return (n - 1) / kMlpChunk + 1; }
 
 struct MlpArgs {
   int n_in, n_out, E;
@@ -18,7 +20,6 @@ struct MlpArgs {
 };
 
 int mlp_param_count(int n_in, int n_out);
-size_t mlp_grad_lds(int n_in, int n_out);
 hipError_t mlp_set_lds_limit(int n_in, int n_out);
 hipError_t launch_mlp_grad(const MlpArgs& a, const float* X, const float* Y, int n, float* partial,
                            float* loss_part, hipStream_t s);

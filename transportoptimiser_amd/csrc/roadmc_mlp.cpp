@@ -22,7 +22,7 @@ namespace {
 
 int mlp_buffers(roadmc_mlp* net, int n) {
   roadmc_ctx* ctx = net->ctx;
-  const int nchunk = (n + 63) / 64;
+  const int nchunk = roadmc::mlp_chunks(n);
   const size_t E = net->a.E;
   int rc;
   if ((rc = rmc_buf_ensure(ctx, net->x, (size_t)n * net->a.n_in * sizeof(float))) ||
@@ -128,7 +128,7 @@ extern "C" int roadmc_mlp_gradient(roadmc_mlp* net, const float* x, const float*
   int rc = mlp_buffers(net, n);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
-  const int nchunk = (n + 63) / 64;
+  const int nchunk = roadmc::mlp_chunks(n);
   RMC_HIP(ctx, hipMemcpyAsync(net->x.ptr, x, (size_t)n * net->a.n_in * sizeof(float),
                               hipMemcpyHostToDevice, s));
   RMC_HIP(ctx, hipMemcpyAsync(net->y.ptr, y, (size_t)n * net->a.n_out * sizeof(float),
@@ -164,7 +164,7 @@ extern "C" int roadmc_mlp_train(roadmc_mlp* net, const float* x, const float* y,
   int rc = mlp_buffers(net, n);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
-  const int nchunk = (n + 63) / 64;
+  const int nchunk = roadmc::mlp_chunks(n);
   RMC_HIP(ctx, hipMemcpyAsync(net->x.ptr, x, (size_t)n * net->a.n_in * sizeof(float),
                               hipMemcpyHostToDevice, s));
   RMC_HIP(ctx, hipMemcpyAsync(net->y.ptr, y, (size_t)n * net->a.n_out * sizeof(float),
