@@ -110,8 +110,8 @@ extern "C" void roadmc_ctx_destroy(roadmc_ctx* ctx) {
                         &ctx->rovs_bufs.blk,  &ctx->rovs_bufs.xs,  &ctx->rovs_bufs.ys,
                         &ctx->rovs_bufs.u,    &ctx->rovs_bufs.small, &ctx->rovs_bufs.grid,
                         &ctx->rovs_bufs.args, &ctx->rovs_bufs.ckpt, &ctx->rovs_bufs.grm,
-                        &ctx->rovs_bufs.rvec, &ctx->rovs_bufs.grids,
-                        &ctx->rovs_grad_bufs.mtpack, &ctx->rovs_grad_bufs.policy,
+                        &ctx->rovs_bufs.rvec, &ctx->rovs_bufs.grids, &ctx->rovs_grad_bufs.mx6,
+                        &ctx->rovs_grad_bufs.mtpack, &ctx->rovs_grad_bufs.mtx6, &ctx->rovs_grad_bufs.policy,
                         &ctx->rovs_grad_bufs.coef, &ctx->rovs_grad_bufs.w,
                         &ctx->rovs_grad_bufs.gpart, &ctx->rovs_grad_bufs.grad,
                         &ctx->rovs_grad_bufs.jpart, &ctx->rovs_grad_bufs.rows,

@@ -90,11 +90,11 @@ struct roadmc_ctx {
         u, small, grid, args, ckpt, grm, rvec, grids;
   } rovs_bufs;
   // The smoothed-validity gradient of the species-state valuation: the
-  // transposed movement matrices, the policy, dJ/dA coefficients, the w
+  // transposed movement matrices and the three-term splits, the policy, dJ/dA coefficients, the w
   // plane, the contraction's partials and result, the per-block values, the
   // rows of each control and the counts that place them.
   struct {
-    rmc_devbuf mtpack, policy, coef, w, gpart, grad, jpart, rows, blk;
+    rmc_devbuf mtpack, mx6, mtx6, policy, coef, w, gpart, grad, jpart, rows, blk;
   } rovs_grad_bufs;
 };
 

@@ -552,9 +552,10 @@ __device__ __forceinline__ uint32_t b6_voff(int nch, int tcol, int lane) {
 // traffic per six MFMAs, against 28 and 3 KB for single tiles.  The B operands
 // of the next chunk are in flight while this chunk's products run; the A
 // operands are split first, then reloaded for the next chunk.
-template <int NR, int NC>
-__device__ __forceinline__ void product_x6(floatx16* acc, const PackedB& B, const float* ap,
-                                           int rstep, const uint32_t* boff, int c0, int c1) {
+// AP: ap(r) is row tile r's operand pointer.
+template <int NR, int NC, class AP>
+__device__ __forceinline__ void product_x6_rows(floatx16* acc, const PackedB& B, const AP& ap,
+                                                const uint32_t* boff, int c0, int c1) {
   floatx16 sm[NR * NC];
 #pragma unroll
   for (int t = 0; t < NR * NC; ++t) acc[t] = sm[t] = floatx16{};
@@ -568,7 +569,7 @@ __device__ __forceinline__ void product_x6(floatx16* acc, const PackedB& B, cons
   auto lda = [&](int c) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-      const floatx4* q = reinterpret_cast<const floatx4*>(ap + r * rstep + 16 * c);
+      const floatx4* q = reinterpret_cast<const floatx4*>(ap(r) + 16 * c);
       a[r][0] = q[0];
       a[r][1] = q[1];
     }
@@ -606,6 +607,13 @@ __device__ __forceinline__ void product_x6(floatx16* acc, const PackedB& B, cons
   if (c < c1) step(b0, b1, c);
 #pragma unroll
   for (int t = 0; t < NR * NC; ++t) acc[t] += sm[t];
+}
+
+// The same with the row tiles at a fixed distance rstep.
+template <int NR, int NC>
+__device__ __forceinline__ void product_x6(floatx16* acc, const PackedB& B, const float* ap,
+                                           int rstep, const uint32_t* boff, int c0, int c1) {
+  product_x6_rows<NR, NC>(acc, B, [&](int r) { return ap + r * rstep; }, boff, c0, c1);
 }
 
 }  // namespace roadmc

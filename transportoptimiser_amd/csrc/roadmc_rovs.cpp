@@ -612,7 +612,9 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
     size_t bytes;
   } need[] = {
       {&B.mpack, (size_t)S * C * Pp * Pk * sizeof(float)},
+      {&G.mx6, (size_t)S * C * Pp * Pk * 6},
       {&G.mtpack, (size_t)S * C * Pp * Pk * sizeof(float)},
+      {&G.mtx6, (size_t)S * C * Pp * Pk * 6},
       {&B.rvec, (size_t)S * C * Pp * sizeof(float)},
       {&B.cols, (size_t)S * 3 * Pp * sizeof(float)},
       {&B.prices, (size_t)(T + 1) * Uc * N * sizeof(double)},
@@ -636,8 +638,7 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
   hipStream_t s = ctx->stream;
 
   // trans o surv_c and its transpose in MFMA B order; the per-patch columns.
-  // The row sums of each origin (for the forward pass's surviving fractions),
-  // at the origin's column of the population tile.
+  // The row sums of each origin (for the forward pass's surviving fractions).
   std::vector<float> mp((size_t)S * C * Pp * Pk, 0.f), mt((size_t)S * C * Pp * Pk, 0.f);
   std::vector<float> cols((size_t)S * 3 * Pp), init_total(S), rvec((size_t)S * C * Pp, 0.f);
   for (int sp = 0; sp < S; ++sp) {
@@ -653,7 +654,7 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
           mt[off + roadmc::mte_pack_index(false, Pk, j, k)] = v;
           rs += v;
         }
-        rvec[((size_t)sp * C + c) * Pp + roadmc::rovs_tile_col(k, false)] = (float)rs;
+        rvec[((size_t)sp * C + c) * Pp + k] = (float)rs;
       }
     }
     float* cl = cols.data() + (size_t)sp * 3 * Pp;
@@ -671,6 +672,11 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
                               hipMemcpyHostToDevice, s));
   RMC_HIP(ctx, hipMemcpyAsync(G.mtpack.ptr, mt.data(), mt.size() * sizeof(float),
                               hipMemcpyHostToDevice, s));
+  RMC_HIP(ctx, roadmc::launch_mte_split_x6(static_cast<const float*>(B.mpack.ptr), mp.size(),
+                                           static_cast<float*>(G.mx6.ptr), s));
+  RMC_HIP(ctx, roadmc::launch_mte_split_x6(static_cast<const float*>(G.mtpack.ptr), mt.size(),
+                                           static_cast<float*>(G.mtx6.ptr), s));
+  const size_t m_species = (size_t)C * Pp * Pk * 3 / 2;  // floats of a species' operands
   RMC_HIP(ctx, hipMemcpyAsync(B.rvec.ptr, rvec.data(), rvec.size() * sizeof(float),
                               hipMemcpyHostToDevice, s));
   RMC_HIP(ctx, hipMemcpyAsync(B.cols.ptr, cols.data(), cols.size() * sizeof(float),
@@ -738,7 +744,7 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
     a.Pp = Pp;
     a.Pk = Pk;
     a.C = C;
-    a.mpack = static_cast<const float*>(B.mpack.ptr) + (size_t)sp * C * Pp * Pk;
+    a.mpack = static_cast<const float*>(G.mx6.ptr) + sp * m_species;
     a.cols = static_cast<const float*>(B.cols.ptr) + (size_t)sp * 3 * Pp;
     for (int i = 0; i < 8; ++i) a.params[i] = pr->species[sp].params[i];
     a.dt = pr->time_step;
@@ -753,14 +759,12 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
     a.aars = static_cast<float*>(B.aars.ptr) + (size_t)sp * T * C * N;
     a.ck = 1;
     a.split = 0;
-    // Controls fixed by the policy: the dots' form (surviving fractions from
-    // the row sums, products only for the controls a tile takes).
     a.rvec = static_cast<const float*>(B.rvec.ptr) + (size_t)sp * C * Pp;
     if (want_grad) {
       a.ckpt = static_cast<float*>(B.ckpt.ptr) + (size_t)sp * T * N * Pp;
       a.grm_out = static_cast<float*>(B.grm.ptr) + (size_t)sp * T * N;
     }
-    RMC_HIP(ctx, roadmc::launch_rovs_forward(a, s));
+    RMC_HIP(ctx, roadmc::launch_rovs_policy_forward(a, s));
   }
 
   // The value and the coefficients dJ_p / dA.
@@ -812,10 +816,8 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
                                        static_cast<int*>(G.rows.ptr), s, true));
 
   // Per species: the reverse sweep, then per control dJ/dM_c = sum over the
-  // years and paths under c of n_t^T w_t (rows in the tile's stored order).
+  // years and paths under c of n_t^T w_t.
   std::vector<double> gm((size_t)Pp * Pp);
-  std::vector<int> pos(P);
-  for (int k = 0; k < P; ++k) pos[k] = roadmc::rovs_tile_col(k, false);
   for (int sp = 0; sp < S; ++sp) {
     const roadmc_rovs_species& sc = pr->species[sp];
     roadmc::RovsAdjArgs a{};
@@ -825,8 +827,8 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
     a.Pp = Pp;
     a.Pk = Pk;
     a.C = C;
-    a.mpack = static_cast<const float*>(B.mpack.ptr) + (size_t)sp * C * Pp * Pk;
-    a.mtpack = static_cast<const float*>(G.mtpack.ptr) + (size_t)sp * C * Pp * Pk;
+    a.mpack = static_cast<const float*>(G.mx6.ptr) + sp * m_species;
+    a.mtpack = static_cast<const float*>(G.mtx6.ptr) + sp * m_species;
     a.cols = static_cast<const float*>(B.cols.ptr) + (size_t)sp * 3 * Pp;
     a.ckpt = static_cast<const float*>(B.ckpt.ptr) + (size_t)sp * T * N * Pp;
     a.grm = static_cast<const float*>(B.grm.ptr) + (size_t)sp * T * N;
@@ -856,7 +858,7 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
       for (int j = 0; j < P; ++j)
         for (int k = 0; k < P; ++k)
           out[(size_t)j * P + k] =
-              sc.trans[(size_t)j * P + k] * gm[(size_t)pos[k] * Pp + j] / (double)N;
+              sc.trans[(size_t)j * P + k] * gm[(size_t)k * Pp + j] / (double)N;
     }
   }
   for (size_t i = 0; i < (size_t)S * C * P * P; ++i)

@@ -40,15 +40,17 @@ struct RovsForwardArgs {
   // Split-bf16 products (mpack in that order, Pk == Pp); the checkpoints then
   // hold each entry's hi | lo << 16 bits.
   int split;
-  // Optional (FP32 only): the row sums of each control's matrix, [C][Pp] in
-  // the tile's column order.  When given, the surviving fractions are dots of
-  // the year-start tile with them, and a tile forms only the products of the
-  // controls its paths take that year (for controls fixed by a policy).
+  // launch_rovs_policy_forward: the row sums of each control's matrix,
+  // [C][Pp]; the surviving fractions are dots of the year-start populations
+  // with them.
   const float* rvec;
 };
 
-size_t rovs_forward_lds(int Pp, int C, bool split, bool dots = false);
 hipError_t launch_rovs_forward(const RovsForwardArgs& a, hipStream_t s);
+// The same for controls fixed by a policy: FP32 products of each path's own
+// control only; mpack is the matrices' three-term split (6 bytes an entry) and
+// the checkpoints are in patch order.
+hipError_t launch_rovs_policy_forward(const RovsForwardArgs& a, hipStream_t s);
 
 // Unit profit per path and year: unit_cost + sum_v fuel_cost_v price_{fuel_idx_v}
 // - unit_revenue sum_c composition_c price_{n_fuels + c}.
@@ -149,17 +151,16 @@ struct RovsSmoothArgs {
 hipError_t launch_rovs_smooth_value(const RovsSmoothArgs& a, hipStream_t s);
 
 // Reverse sweep of one species' populations under the policy, years T-1 .. 0,
-// one 32-path tile per workgroup: x_t = n_t M_u (every control's product, the
-// path's selected), w_t = lambda_t+1 o G'(x_t) + coef_t on the patches (zero
+// x_t = n_t M_u, w_t = lambda_t+1 o G'(x_t) + coef_t on the patches (zero
 // on padding), lambda_t = w_t M_u^T; w_t goes to w_out for dJ/dM_c = sum over
-// (t, paths with u = c) of n_t^T w_t.  FP32 products on the forward pass's
-// packed operands.
+// (t, paths with u = c) of n_t^T w_t.  FP32 products, three-term
+// split operands as the forward pass's.
 struct RovsAdjArgs {
   int N, T, P, Pp, Pk, C;
   const float* mpack;     // [C][Pp * Pk] trans o surv_c, MFMA B order
   const float* mtpack;    // [C][Pp * Pk] its transpose, same order
   const float* cols;      // [3][Pp]: K, 1/K, initial population
-  const float* ckpt;      // [T][N][Pp] populations entering each year, tile order
+  const float* ckpt;      // [T][N][Pp] populations entering each year
   const float* grm;       // [T][N] growth-rate means of each year's growth
   const int* policy;      // [T][N]
   const float* coef;      // [T][N] this species' dJ_p / dA_t
@@ -167,7 +168,6 @@ struct RovsAdjArgs {
   uint32_t tag0, key0, key1;
   float* w_out;           // [T][N][Pp]
 };
-size_t rovs_adj_lds(int Pp);
 hipError_t launch_rovs_adj(const RovsAdjArgs& a, hipStream_t s);
 
 // Lists of the n rows of ctl [n] by control, stable.  First call (scatter

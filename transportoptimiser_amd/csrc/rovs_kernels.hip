@@ -22,9 +22,9 @@
 //     waves), each path's own control kept by a register select, then the
 //     growth-rate SDE and the logistic growth with the reference's /100 in
 //     the epilogue, noise from Philox in registers.  Under controls fixed by
-//     a policy (the smoothed gradient), a second form takes the AARs as dots
-//     of the year-start tile with each control's row sums and forms only the
-//     products of the controls the tile's paths take;
+//     a policy (the smoothed gradient), rovs_policy_kernel takes the AARs as
+//     dots of the year-start tile with each control's row sums and multiplies
+//     each path by its own control's matrix only;
 //   - per backward step: one kernel forms the states and counts each
 //     control's included paths per block, one scans the counts, one
 //     scatters the samples in path order (so that kNN ties resolve as in a
@@ -103,16 +103,14 @@ constexpr int rovs_min_waves() {
 
 static int rovs_pad(bool split) { return split ? TraitsB3::PAD : TF::PAD; }
 
-size_t rovs_forward_lds(int Pp, int C, bool split, bool dots) {
+size_t rovs_forward_lds(int Pp, int C, bool split) {
   const int LDA = Pp + rovs_pad(split);
   return (size_t)kRovsRows * LDA * sizeof(float)      // state tile
          + kRovsRows * sizeof(float)                  // growth-rate means
          + (size_t)rovs_waves(Pp) * kRovsRows * sizeof(float)  // per-wave row sums
          + kRovsRows * sizeof(float)                  // row totals
          + (size_t)C * kRovsRows * sizeof(float)      // AARs
-         + kRovsRows * sizeof(int)                    // controls
-         // the dots' partial sums: 2 strides of columns per wave
-         + (dots ? (size_t)2 * rovs_waves(Pp) * C * kRovsRows * sizeof(float) : 0);
+         + kRovsRows * sizeof(int);                   // controls
 }
 
 // Sum over the 32 columns held by the 32 lanes of a half-wave.
@@ -140,10 +138,7 @@ __device__ __forceinline__ void rovs_product(floatx16* acc, const PackedB& B, co
   }
 }
 
-// DOTS: the surviving fractions from dots with a.rvec and products only for
-// the controls the tile's paths take (a.rvec given); otherwise from the row
-// sums of every control's product.
-template <class TR, bool DOTS>
+template <class TR>
 __global__ __launch_bounds__(kRovsMaxThreads)
 __attribute__((amdgpu_waves_per_eu(rovs_min_waves<TR>()))) void rovs_forward_kernel(
     RovsForwardArgs a) {
@@ -159,8 +154,6 @@ __attribute__((amdgpu_waves_per_eu(rovs_min_waves<TR>()))) void rovs_forward_ker
   float* tot = rsum + NW * kRovsRows;
   float* aar = tot + kRovsRows;     // [C][32]
   int* ctl = reinterpret_cast<int*>(aar + C * kRovsRows);
-  const int nq = nthreads / kRovsRows;                   // column strides of the dots
-  float* spart = reinterpret_cast<float*>(ctl + kRovsRows);  // [nq][C][32] (DOTS)
   const float* K = a.cols;
   const float* Kinv = a.cols + Pp;
   const float* init = a.cols + 2 * Pp;
@@ -210,52 +203,15 @@ __attribute__((amdgpu_waves_per_eu(rovs_min_waves<TR>()))) void rovs_forward_ker
       }
     }
     __syncthreads();
-    unsigned used = ~0u;
-    if constexpr (DOTS) {
-      // The surviving fractions' numerators as dots of the year-start tile
-      // with each control's row sums (a stride of columns per thread, summed
-      // over the strides in order after the products), and the controls some
-      // path of the tile takes (the same mask in every wave).
-      const int r = tid & (kRovsRows - 1), q = tid / kRovsRows;
-      const RovsTile<TR> ts{A, LDAy};
-      float accs[kRovsMaxC];
-#pragma unroll
-      for (int c = 0; c < kRovsMaxC; ++c) accs[c] = 0.f;
-      for (int i = q; i < Pp; i += nq) {
-        const float v = ts.get(r, i);
-#pragma unroll
-        for (int c = 0; c < kRovsMaxC; ++c)
-          if (c < C) accs[c] += v * a.rvec[(size_t)c * Pp + i];
-      }
-#pragma unroll
-      for (int c = 0; c < kRovsMaxC; ++c)
-        if (c < C) spart[(q * C + c) * kRovsRows + r] = accs[c];
-      used = 0u;
-      const int cl = laney < kRovsRows ? ctl[laney] : -1;
-      for (int c = 0; c < C; ++c)
-        if (__ballot(cl == c) != 0ull) used |= 1u << c;
-    }
     floatx16 sel[kRovsNT], acc[kRovsNT];
 #pragma unroll
     for (int t = 0; t < kRovsNT; ++t) sel[t] = floatx16{};
     for (int c = 0; c < C; ++c) {
-      if (!((used >> c) & 1u)) continue;
       const PackedB B = packed_b(a.mpack + (size_t)c * Pp * a.Pk, nkg, mbytes);
       if (my_n == 1)
         rovs_product<TR, 1>(acc, B, A, tcol, LDAy, arow, akoff, laney);
       else if (my_n == 2)
         rovs_product<TR, 2>(acc, B, A, tcol, LDAy, arow, akoff, laney);
-      if constexpr (DOTS) {
-        // The select of each path's own control only.
-#pragma unroll
-        for (int r = 0; r < TF::NACC; ++r)
-          if (ctl[TF::acc_row(laney, r)] == c) {
-#pragma unroll
-            for (int t = 0; t < kRovsNT; ++t)
-              if (t < my_n) sel[t][r] = acc[t][r];
-          }
-        continue;
-      }
       // Row sums of this control's product over the wave's columns, and the
       // select of each path's own control.
 #pragma unroll
@@ -292,15 +248,7 @@ __attribute__((amdgpu_waves_per_eu(rovs_min_waves<TR>()))) void rovs_forward_ker
       grm[tid] = g + rev * (mu - g) * dt + g * (zb * sd) + (__expf(jsz) - 1.f) * g * jump;
       if (a.grm_out && p0 + tid < a.N) a.grm_out[(size_t)year * a.N + p0 + tid] = grm[tid];
     }
-    __syncthreads();  // (DOTS: also every wave's products have read the tile)
-    if constexpr (DOTS) {
-      if (tid < C * kRovsRows) {
-        const int c = tid / kRovsRows, r = tid - c * kRovsRows;
-        float sm = 0.f;
-        for (int qq = 0; qq < nq; ++qq) sm += spart[(qq * C + c) * kRovsRows + r];
-        aar[c * kRovsRows + r] = sm / tot[r];
-      }
-    }
+    __syncthreads();
     // Growth (SimulateGPU.cu:902-916): g = grMean + z lv per patch,
     // n = n' (1 + g (K - n') / K / 100), written back to the tile.
     int LDAe = LDA, p0e = p0, lanee = lane;
@@ -353,30 +301,21 @@ __attribute__((amdgpu_waves_per_eu(rovs_min_waves<TR>()))) void rovs_forward_ker
   }
 }
 
-template <class TR, bool DOTS>
+template <class TR>
 static hipError_t launch_rovs_forward_t(const RovsForwardArgs& a, hipStream_t s) {
-  const size_t lds = rovs_forward_lds(a.Pp, a.C, TR::kSplit, DOTS);
-  hipError_t e =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&rovs_forward_kernel<TR, DOTS>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const size_t lds = rovs_forward_lds(a.Pp, a.C, TR::kSplit);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&rovs_forward_kernel<TR>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   const int blocks = (a.N + kRovsRows - 1) / kRovsRows;
-  hipLaunchKernelGGL((rovs_forward_kernel<TR, DOTS>), dim3(blocks), dim3(64 * rovs_waves(a.Pp)),
-                     lds, s, a);
+  hipLaunchKernelGGL(rovs_forward_kernel<TR>, dim3(blocks), dim3(64 * rovs_waves(a.Pp)), lds, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_rovs_forward(const RovsForwardArgs& a, hipStream_t s) {
   // Split-bf16 products contract over Pp (an even count of 16-k chunks).
   if (a.split && a.Pk != a.Pp) return hipErrorInvalidValue;
-  if (a.rvec) {
-    // The dots' form: FP32 products, at most kRovsMaxC controls (C x 32 <= 256
-    // threads finish the sums).
-    if (a.split || a.C < 1 || a.C > kRovsMaxC) return hipErrorInvalidValue;
-    return launch_rovs_forward_t<TF, true>(a, s);
-  }
-  return a.split ? launch_rovs_forward_t<TraitsB3, false>(a, s)
-                 : launch_rovs_forward_t<TF, false>(a, s);
+  return a.split ? launch_rovs_forward_t<TraitsB3>(a, s) : launch_rovs_forward_t<TF>(a, s);
 }
 
 // Unit profit (computePathStates, SimulateGPU.cu:985-1002) with the ore
@@ -1024,143 +963,483 @@ hipError_t launch_rovs_smooth_value(const RovsSmoothArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-size_t rovs_adj_lds(int Pp) {
-  return (size_t)kRovsRows * (Pp + TF::PAD) * sizeof(float)  // population, then w, tile
-         + 2 * kRovsRows * sizeof(float)                     // growth-rate means, coefficients
-         + kRovsRows * sizeof(int);                          // controls of the year
+// ---- Under a policy: rows grouped by control -----------------------------------
+//
+// A workgroup of eight waves holds BM (8 to 160) paths of a species in LDS
+// (FP32, natural column order).  A year moves every path by its own control's
+// matrix.  Forming every control's product for every path and keeping one
+// costs C products; instead the rows are grouped by control (a stable
+// compaction into groups padded to the 32 rows of a product tile) and each
+// group multiplies its own control's matrix: the operand reads take their row
+// from the group's map, so nothing moves in LDS.  At 128 paths and 3 controls
+// that is about 6 row tiles instead of 12, and each B operand serves the two
+// tiles of its group.  A wave owns one column tile (two above 256 patches)
+// and keeps its products of all groups in registers until every wave has read
+// the tile; they are then written to the paths' rows, and a second pass over
+// the tile applies the growth with one Philox call per four paths, lanes along
+// the columns (the groups' rows are not path quads).  The products are those
+// of the MTE kernels (TraitsX6).
+// The surviving fractions under every control are dots of the year-start rows
+// with the matrices' row sums, sixteen interleaved FP32 sums per row.
+// The valuations keep the FP32 MFMA of every control: their backward passes
+// amplify the populations' last digits (a changed neighbour set or decision
+// moved the value by up to 2%), which the smoothed value does not.
+// At P = 256, C = 3, N = 100,000, T = 50: forward 8.8 ms, reverse
+// sweep 16.0 ms (20.7 and 34.6 ms with 32-path tiles on the FP32 MFMA, every
+// control a tile uses multiplied and each path's product selected).
+constexpr int kRgWaves = 8, kRgThreads = kRgWaves * 64;
+constexpr int kRgTiles = 7;  // group tiles at most
+constexpr int kRgMaxRows = 160;
+constexpr int kRgParts = 4;  // column quarters of a row's dots
+
+// Column tiles a wave owns, and the group tiles whose products it can hold:
+// 7 (an eighth spills in the product loop) or 4 of two columns.
+static int rg_cols(int Pp) { return Pp > 32 * kRgWaves ? 2 : 1; }
+__host__ __device__ constexpr int rg_slots(int cols) { return cols == 1 ? kRgTiles : 4; }
+
+// Group tiles that BM rows under C controls can need.
+static int rg_max_tiles(int BM, int C) { return (BM - std::min(C, BM)) / 32 + std::min(C, BM); }
+
+struct RgPlan {
+  int BM;
+  int dense;  // 32 rows, every used control's product, selected per path
+  size_t lds;
+};
+
+// LDS: n_tiles tiles, then [kRgParts][C + 1][BM] partial dots, [n_st][C + 1][BM]
+// dots, growth-rate means, totals or coefficients, controls, the row map
+// ([kRgTiles][32]) and the tiles' controls.
+static size_t rg_lds(int BM, int Pp, int C, int n_tiles, int n_st) {
+  return sizeof(float) * ((size_t)n_tiles * BM * (Pp + TraitsX6::PAD) +
+                          (size_t)(kRgParts + n_st) * (C + 1) * BM + 3 * (size_t)BM + kRgTiles * 32 + 16);
 }
 
-// Reverse sweep of one species under the policy (RovsAdjArgs).  lambda stays
-// in the accumulator layout of the wave's column tiles from year to year: the
-// tile assignment of the two products is the same, so each lane keeps the
-// entries it needs for the next year's w.
-// Three waves per SIMD, as the FP32 forward pass (168 VGPRs, a few spilled).
-__global__ __launch_bounds__(kRovsMaxThreads) __attribute__((amdgpu_waves_per_eu(3))) void
-rovs_adj_kernel(RovsAdjArgs a) {
-  constexpr int NT = kRovsNT;
-  extern __shared__ char smem[];
+// The rows of a launch over N paths: of the sizes (whole path quads) that LDS
+// and the waves' registers allow, the one with the least rounds of workgroups
+// over the CUs times work, in product tiles: 1.6 for 32 paths (product, growth
+// and dots) and half a tile of padding per control.  The results do not depend
+// on the rows.
+static RgPlan rg_plan(int N, int Pp, int C, int n_tiles, int n_st) {
+  constexpr size_t kLdsMax = 160 * 1024;
+  constexpr int kCus = 256;
+  RgPlan best{32, 0, rg_lds(32, Pp, C, n_tiles, n_st)};
+  best.dense = rg_max_tiles(8, C) > rg_slots(rg_cols(Pp));
+  double cost = 1e300;
+  for (int BM = 8; BM <= kRgMaxRows; BM += 4) {
+    const size_t lds = rg_lds(BM, Pp, C, n_tiles, n_st);
+    if (lds > kLdsMax || rg_max_tiles(BM, C) > rg_slots(rg_cols(Pp))) continue;
+    const int rounds = ((N + BM - 1) / BM + kCus - 1) / kCus;
+    const double c = rounds * (1.6 * BM / 32 + 0.5 * C);
+    if (c < cost) {
+      cost = c;
+      best = RgPlan{BM, 0, lds};
+    }
+  }
+  return best;
+}
+
+struct RgShape {
+  int BM, Pp, LDA, nch, C, dense;
+};
+
+// A fresh copy of the lane number, so that the addresses and columns derived
+// from it are computed again where they are used instead of being kept, and
+// spilled, over the year loop.
+__device__ __forceinline__ void rg_opaque(int* lane) { asm volatile("" : "+v"(*lane)); }
+
+// Wave 0: map [tile][32] holds the row of each group slot (-1 in the padding),
+// tiles[t] the control of group tile t and tiles[kRgTiles] their number.  ctl
+// is -1 for rows past the last path.
+__device__ __forceinline__ void rg_group(const RgShape& sh, const int* ctl, int* map, int* tiles,
+                                         int lane) {
+#pragma unroll
+  for (int i = 0; i < kRgTiles * 32; i += 64)
+    if (i + lane < kRgTiles * 32) map[i + lane] = -1;
+  const int c0 = lane < sh.BM ? ctl[lane] : -1;
+  const int c1 = 64 + lane < sh.BM ? ctl[64 + lane] : -1;
+  const int c2 = 128 + lane < sh.BM ? ctl[128 + lane] : -1;
+  const uint64_t below = (1ull << lane) - 1;
+  int nt = 0;
+  for (int c = 0; c < sh.C; ++c) {
+    const uint64_t m0 = __ballot(c0 == c), m1 = __ballot(c1 == c), m2 = __ballot(c2 == c);
+    const int n0 = __popcll(m0), n1 = n0 + __popcll(m1), n = n1 + __popcll(m2);
+    if (c0 == c) map[32 * nt + __popcll(m0 & below)] = lane;
+    if (c1 == c) map[32 * nt + n0 + __popcll(m1 & below)] = 64 + lane;
+    if (c2 == c) map[32 * nt + n1 + __popcll(m2 & below)] = 128 + lane;
+    const int k = (n + 31) >> 5;
+    if (lane < k) tiles[nt + lane] = c;
+    nt += k;
+  }
+  if (lane == 0) tiles[kRgTiles] = nt;
+}
+
+// Replaces each path's row of the tile by its product with its control's
+// matrix (mx6: C matrices packed for TraitsX6, mbytes each).  Every thread of
+// the workgroup calls it; it ends with a barrier.
+template <int NCW>
+__device__ __forceinline__ void rg_move(const RgShape& sh, float* A, const char* mx6,
+                                        size_t mbytes, const int* ctl, const int* map,
+                                        const int* tiles, int wave, int lane) {
+  constexpr int SL = rg_slots(NCW);
+  rg_opaque(&lane);
+  const int ntc = sh.Pp >> 5, wpc = NCW == 1 ? kRgWaves / ntc : 1;
+  const int sub = NCW == 1 ? wave / ntc : 0, col0 = NCW == 1 ? wave - sub * ntc : wave;
+  const int akoff = 8 * (lane >> 5);
+  floatx16 acc[NCW][SL];
+  int base = 0, end = 0;
+  if (!sh.dense) {
+    const int nt = __builtin_amdgcn_readfirstlane(tiles[kRgTiles]);
+    const int per = (nt + wpc - 1) / wpc;
+    base = sub * per;
+    end = sub < wpc ? min(nt, base + per) : base;
+#pragma unroll
+    for (int j = 0; j < NCW; ++j) {
+      const int col = col0 + kRgWaves * j;
+      if (col >= ntc) continue;
+      const uint32_t bo = b6_voff(sh.nch, col, lane);
+      auto rows = [&](int s) -> const float* {
+        return A + max(map[32 * s + (lane & 31)], 0) * sh.LDA + akoff;
+      };
+      auto matrix = [&](int c) {
+        return packed_b(mx6 + (size_t)c * mbytes, 0, mbytes);
+      };
+#pragma unroll
+      for (int i = 0; i < SL; i += 2) {
+        const int s = base + i;
+        if (s >= end) continue;
+        const int ca = __builtin_amdgcn_readfirstlane(tiles[s]);
+        const float* const a0 = rows(s);
+        if (i + 1 < SL) {
+          const int cb = s + 1 < end ? __builtin_amdgcn_readfirstlane(tiles[s + 1]) : -1;
+          if (ca == cb) {
+            const float* const a1 = rows(s + 1);
+            product_x6_rows<2, 1>(&acc[j][i], matrix(ca), [&](int r) { return r ? a1 : a0; }, &bo,
+                                  0, sh.nch);
+            continue;
+          }
+          if (cb >= 0) product_x6<1, 1>(&acc[j][i + 1], matrix(cb), rows(s + 1), 0, &bo, 0, sh.nch);
+        }
+        product_x6<1, 1>(&acc[j][i], matrix(ca), a0, 0, &bo, 0, sh.nch);
+      }
+    }
+  } else {
+    // 32 rows: every control that some path takes, selected per path.
+    const int cl = lane < 32 ? ctl[lane] : -1;
+    const float* const a0 = A + (lane & 31) * sh.LDA + akoff;
+#pragma unroll
+    for (int j = 0; j < NCW; ++j) {
+      const int col = col0 + kRgWaves * j;
+      acc[j][0] = floatx16{};
+      if (sub > 0 || col >= ntc) continue;
+      const uint32_t bo = b6_voff(sh.nch, col, lane);
+      for (int c = 0; c < sh.C; ++c) {
+        if (__ballot(cl == c) == 0ull) continue;
+        floatx16 t;
+        product_x6<1, 1>(&t, packed_b(mx6 + (size_t)c * mbytes, 0, mbytes), a0, 0, &bo, 0, sh.nch);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (ctl[TraitsX6::acc_row(lane, r)] == c) acc[j][0][r] = t[r];
+      }
+    }
+    base = 0;
+    end = sub == 0 ? 1 : 0;
+  }
+  __syncthreads();  // every wave has read the tile
+#pragma unroll
+  for (int j = 0; j < NCW; ++j) {
+    const int col = col0 + kRgWaves * j;
+    if (col >= ntc) continue;
+    float* const Ac = A + 32 * col + (lane & 31);
+#pragma unroll
+    for (int i = 0; i < SL; ++i) {
+      if (base + i >= end) continue;
+#pragma unroll
+      for (int r4 = 0; r4 < 16; r4 += 4) {
+        const int g = 32 * (base + i) + TraitsX6::acc_row(lane, r4);
+        int4 m;
+        if (sh.dense)
+          m = make_int4(g, g + 1, g + 2, g + 3);
+        else
+          m = *reinterpret_cast<const int4*>(map + g);
+        if (m.x >= 0) Ac[m.x * sh.LDA] = acc[j][i][r4];
+        if (m.y >= 0) Ac[m.y * sh.LDA] = acc[j][i][r4 + 1];
+        if (m.z >= 0) Ac[m.z * sh.LDA] = acc[j][i][r4 + 2];
+        if (m.w >= 0) Ac[m.w * sh.LDA] = acc[j][i][r4 + 3];
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// fn(quad row, column, capacity, 1 / capacity, z[4]) over the tile's path
+// quads and columns, lanes along the columns; z are the quad's patch normals.
+template <class F>
+__device__ __forceinline__ void rg_quads(const RgShape& sh, const float* cols, int p0, int year,
+                                         uint32_t tag0, uint32_t key0, uint32_t key1, int wave,
+                                         int lane, const F& fn) {
+  rg_opaque(&lane);
+  const int ncb = (sh.Pp + 63) >> 6, parts = kRgWaves / ncb;
+  const int part = wave / ncb, col = (wave - part * ncb) * 64 + lane;
+  if (part >= parts || col >= sh.Pp) return;
+  const float K = cols[col], Ki = cols[sh.Pp + col];
+  const int nq = sh.BM >> 2, q1 = nq * (part + 1) / parts;
+  for (int q = nq * part / parts; q < q1; ++q) {
+    float z[4];
+    TraitsX6::normal4((uint32_t)(p0 + 4 * q) >> 2, (uint32_t)year, (uint32_t)col, tag0, key0, key1,
+                      z);
+    fn(4 * q, col, K, Ki, z);
+  }
+}
+
+// Growth (SimulateGPU.cu:902-916): g = grMean + z lv per patch, n = n' (1 + g
+// (K - n') / K / 100).
+__device__ __forceinline__ void rg_grow(const RgShape& sh, float* A, const float* cols,
+                                        const float* grm, float lv, int p0, int year,
+                                        uint32_t tag0, uint32_t key0, uint32_t key1, int wave,
+                                        int lane) {
+  rg_quads(sh, cols, p0, year, tag0, key0, key1, wave, lane,
+           [&](int row, int col, float K, float Ki, const float* z) {
+             float* a = A + row * sh.LDA + col;
+             const float4 gm = *reinterpret_cast<const float4*>(grm + row);
+             const float g[4] = {gm.x + z[0] * lv, gm.y + z[1] * lv, gm.z + z[2] * lv,
+                                 gm.w + z[3] * lv};
+#pragma unroll
+             for (int s = 0; s < 4; ++s) {
+               const float x = a[s * sh.LDA];
+               a[s * sh.LDA] = x * (1.f + g[s] * (K - x) * Ki * 0.01f);
+             }
+           });
+}
+
+// Partial dots of each row: part[q][0][row] its total and part[q][1 + c][row]
+// its product with rvec[c] over column quarter q, in four interleaved sums.
+// A wave takes 64 rows and a quarter, so the columns are uniform and rvec comes
+// through scalar loads (lane-held columns: 20,000 cycles a year at 132 paths of
+// 256 patches, all of it the loads' latency).  rg_dots_sum adds the quarters in
+// order after a barrier.
+template <int CC>
+__device__ __forceinline__ void rg_dots_c(const RgShape& sh, const float* A, int C,
+                                          const float* rvec, float* part, int wave, int lane) {
+  typedef const __attribute__((address_space(4))) floatx4 ConstX4;
+  rg_opaque(&lane);
+  const int groups = (sh.BM + 63) >> 6, n = sh.Pp >> 4;  // float4s of a quarter
+  for (int it = wave; it < groups * kRgParts; it += kRgWaves) {
+    const int q = it & (kRgParts - 1), row = (it / kRgParts) * 64 + lane;
+    const int r = min(row, sh.BM - 1);
+    ConstX4* w[CC + 1];
+#pragma unroll
+    for (int c = 0; c < CC; ++c)
+      w[c] = (ConstX4*)(uintptr_t)(rvec + (size_t)min(c, C - 1) * sh.Pp) + q * n;
+    const floatx4* v4 = reinterpret_cast<const floatx4*>(A + r * sh.LDA) + q * n;
+    floatx4 t = {}, d[CC + 1];
+#pragma unroll
+    for (int c = 0; c < CC; ++c) d[c] = floatx4{};
+#pragma unroll 2
+    for (int i = 0; i < n; ++i) {
+      const floatx4 v = v4[i];
+      t += v;
+#pragma unroll
+      for (int c = 0; c < CC; ++c) {
+        const floatx4 x = w[c][i];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[c][k] = fmaf(v[k], x[k], d[c][k]);
+      }
+    }
+    auto sum = [](const floatx4& v) { return (v[0] + v[1]) + (v[2] + v[3]); };
+    if (row < sh.BM) {
+      float* o = part + (size_t)q * (C + 1) * sh.BM + row;
+      o[0] = sum(t);
+#pragma unroll
+      for (int c = 0; c < CC; ++c)
+        if (c < C) o[(1 + c) * sh.BM] = sum(d[c]);
+    }
+  }
+}
+__device__ __forceinline__ void rg_dots(const RgShape& sh, const float* A, int C,
+                                        const float* rvec, float* part, int wave, int lane) {
+  if (C == 0)
+    rg_dots_c<0>(sh, A, C, rvec, part, wave, lane);
+  else if (C <= 4)
+    rg_dots_c<4>(sh, A, C, rvec, part, wave, lane);
+  else
+    rg_dots_c<kRovsMaxC>(sh, A, C, rvec, part, wave, lane);
+}
+
+__device__ __forceinline__ void rg_dots_sum(const RgShape& sh, int C, const float* part, float* st,
+                                            int tid) {
+  const int n = (C + 1) * sh.BM;
+  for (int i = tid; i < n; i += kRgThreads)
+    st[i] = (part[i] + part[n + i]) + (part[2 * n + i] + part[3 * n + i]);
+}
+
+// The tile's rows from or to [N][Pp] rows in HBM, a wave to a row.
+__device__ __forceinline__ void rg_load(const RgShape& sh, float* A, const float* src, int p0,
+                                        int N, int wave, int lane) {
+  for (int r = wave; r < sh.BM; r += kRgWaves)
+    for (int c = 4 * lane; c < sh.Pp; c += 256)
+      *reinterpret_cast<floatx4*>(A + r * sh.LDA + c) =
+          p0 + r < N ? *reinterpret_cast<const floatx4*>(src + (size_t)(p0 + r) * sh.Pp + c)
+                     : floatx4{};
+}
+__device__ __forceinline__ void rg_store(const RgShape& sh, const float* A, float* dst, int p0,
+                                         int N, int wave, int lane) {
+  for (int r = wave; r < sh.BM; r += kRgWaves)
+    for (int c = 4 * lane; c < sh.Pp && p0 + r < N; c += 256)
+      *reinterpret_cast<floatx4*>(dst + (size_t)(p0 + r) * sh.Pp + c) =
+          *reinterpret_cast<const floatx4*>(A + r * sh.LDA + c);
+}
+
+// LDS arrays after the tiles.
+struct RgArrays {
+  float *part, *st, *grm, *aux;
+  int *ctl, *map, *tiles;
+};
+__device__ __forceinline__ RgArrays rg_arrays(const RgShape& sh, float* smem, int n_tiles,
+                                              int n_st) {
+  RgArrays r;
+  r.part = smem + (size_t)n_tiles * sh.BM * sh.LDA;
+  r.st = r.part + kRgParts * (sh.C + 1) * sh.BM;
+  r.grm = r.st + n_st * (sh.C + 1) * sh.BM;
+  r.aux = r.grm + sh.BM;
+  r.ctl = reinterpret_cast<int*>(r.aux + sh.BM);
+  r.map = r.ctl + sh.BM;
+  r.tiles = r.map + kRgTiles * 32;
+  return r;
+}
+
+template <int NCW>
+__global__ __launch_bounds__(kRgThreads) void rovs_policy_kernel(RovsForwardArgs a, int BM,
+                                                                     int dense) {
+  extern __shared__ __attribute__((aligned(16))) float rg_smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nthreads = blockDim.x, NW = nthreads >> 6;
-  const int Pp = a.Pp, LDA = Pp + TF::PAD, C = a.C, N = a.N;
-  const int p0 = blockIdx.x * kRovsRows;
-  float* A = reinterpret_cast<float*>(smem);
-  float* gm = A + kRovsRows * LDA;
-  float* cf = gm + kRovsRows;
-  int* ctl = reinterpret_cast<int*>(cf + kRovsRows);
-  const float* K = a.cols;
-  const float* Kinv = a.cols + Pp;
-  const int ntc = Pp / TF::TN;
-  const int base = ntc / NW, extra = ntc % NW;
-  const int my_n = base + (wave < extra ? 1 : 0);
-  const int my_t0 = wave * base + (wave < extra ? wave : extra);
-  int tcol[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) tcol[t] = my_t0 + t;
-  const int arow = TF::a_row(lane), akoff = TF::KV * TF::k_lane(lane);
-  const int nkg = a.Pk >> 3;
-  const size_t mbytes = (size_t)Pp * a.Pk * sizeof(float);
-  floatx16 lam[NT], sel[NT], acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) lam[t] = floatx16{};
-
-  for (int year = a.T - 1; year >= 0; --year) {
-    // The tile entering the year (stored positions, as the forward pass
-    // wrote it), the year's controls, coefficients and growth-rate means.
-    const float* src = a.ckpt + (size_t)year * N * Pp;
-    for (int idx = tid; idx < kRovsRows * Pp; idx += nthreads) {
-      const int r = idx / Pp, c = idx - r * Pp;
-      A[r * LDA + c] = (p0 + r < N) ? src[(size_t)(p0 + r) * Pp + c] : 0.f;
+  const RgShape sh{BM, a.Pp, a.Pp + TraitsX6::PAD, a.Pk >> 4, a.C, dense};
+  const int p0 = blockIdx.x * BM, C = a.C, N = a.N;
+  float* const A = rg_smem;
+  const RgArrays L = rg_arrays(sh, rg_smem, 1, 1);
+  const float mu = (float)a.params[1], sd = (float)a.params[2], rev = (float)a.params[4];
+  const float jmp = (float)a.params[5], jprob = (float)a.params[6], lv = (float)a.params[7];
+  const float dt = (float)a.dt;
+  const size_t mbytes = (size_t)a.Pp * a.Pk * 6;
+  const float* init = a.cols + 2 * a.Pp;
+  for (int r = wave; r < BM; r += kRgWaves)
+    for (int c = lane; c < a.Pp; c += 64) A[r * sh.LDA + c] = init[c];
+  if (tid < BM) {
+    L.grm[tid] = (float)a.params[0];
+    if (p0 + tid < N) a.total_pops[p0 + tid] = a.init_total;
+  }
+  __syncthreads();
+  for (int year = 0; year < a.T; ++year) {
+    rg_dots(sh, A, C, a.rvec, L.part, wave, lane);
+    if (tid < BM) {
+      const bool in = p0 + tid < N;
+      L.ctl[tid] = in ? a.controls[(size_t)year * N + p0 + tid] : -1;
+      // Growth-rate SDE per path (SimulateGPU.cu:839-851), jump probability
+      // from its own field.
+      float zb, zj, uj;
+      path_scalars<float>((uint32_t)(p0 + tid), (uint32_t)year, a.tag1, a.key0, a.key1, &zb, &zj,
+                          &uj);
+      const float g = L.grm[tid];
+      const float jump = (uj < jprob) ? 1.f : 0.f;
+      const float jsz = zj * jmp * jmp - jmp * jmp / 2.f;
+      const float gn = g + rev * (mu - g) * dt + g * (zb * sd) + (__expf(jsz) - 1.f) * g * jump;
+      L.grm[tid] = gn;
+      if (a.grm_out && in) a.grm_out[(size_t)year * N + p0 + tid] = gn;
     }
-    if (tid < kRovsRows) {
+    // Checkpoint of the tile at the start of the year.
+    if (a.ckpt && year % a.ck == 0)
+      rg_store(sh, A, a.ckpt + (size_t)(year / a.ck) * N * a.Pp, p0, N, wave, lane);
+    __syncthreads();
+    if (wave == 0) rg_group(sh, L.ctl, L.map, L.tiles, lane);
+    rg_dots_sum(sh, C, L.part, L.st, tid);
+    __syncthreads();
+    if (tid < BM && p0 + tid < N) {
+      const float tot = year ? L.st[tid] : a.init_total;
+      if (year) a.total_pops[(size_t)year * N + p0 + tid] = tot;
+      for (int c = 0; c < C; ++c)
+        a.aars[((size_t)year * C + c) * N + p0 + tid] = L.st[(1 + c) * BM + tid] / tot;
+    }
+    rg_move<NCW>(sh, A, reinterpret_cast<const char*>(a.mpack), mbytes, L.ctl, L.map, L.tiles, wave,
+                 lane);
+    rg_grow(sh, A, a.cols, L.grm, lv, p0, year, a.tag0, a.key0, a.key1, wave, lane);
+    __syncthreads();
+  }
+  rg_dots(sh, A, 0, nullptr, L.part, wave, lane);
+  __syncthreads();
+  rg_dots_sum(sh, 0, L.part, L.st, tid);
+  __syncthreads();
+  if (tid < BM && p0 + tid < N) a.total_pops[(size_t)a.T * N + p0 + tid] = L.st[tid];
+}
+
+// Launches fn(args, rows, dense) over the paths.
+template <class Args>
+static hipError_t rg_launch(const RgPlan& pl, const void* fn, const Args& a, hipStream_t s) {
+  if (pl.lds > 160 * 1024) return hipErrorInvalidValue;
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds);
+  if (e != hipSuccess) return e;
+  Args arg = a;
+  int BM = pl.BM, dense = pl.dense;
+  void* args[] = {&arg, &BM, &dense};
+  e = hipLaunchKernel(fn, dim3((a.N + BM - 1) / BM), dim3(kRgThreads), args, pl.lds, s);
+  return e != hipSuccess ? e : hipGetLastError();
+}
+
+// Reverse sweep of one species under the policy (RovsAdjArgs): the rows
+// grouped as in the forward pass, one tile for n_t, x_t, w_t and lambda_t in
+// turn and one for lambda_t+1.
+template <int NCW>
+__global__ __launch_bounds__(kRgThreads) void rovs_adj_kernel(RovsAdjArgs a, int BM, int dense) {
+  extern __shared__ __attribute__((aligned(16))) float rg_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const RgShape sh{BM, a.Pp, a.Pp + TraitsX6::PAD, a.Pk >> 4, a.C, dense};
+  const int p0 = blockIdx.x * BM, N = a.N, Pp = a.Pp;
+  const RgArrays L = rg_arrays(sh, rg_smem, 2, 1);
+  const size_t mbytes = (size_t)Pp * a.Pk * 6;
+  float *X = rg_smem, *Y = rg_smem + (size_t)BM * sh.LDA;
+  for (int i = tid; i < BM * sh.LDA; i += kRgThreads) Y[i] = 0.f;
+  for (int year = a.T - 1; year >= 0; --year) {
+    rg_load(sh, X, a.ckpt + (size_t)year * N * Pp, p0, N, wave, lane);
+    if (tid < BM) {
       const bool in = p0 + tid < N;
       const size_t at = (size_t)year * N + p0 + tid;
-      ctl[tid] = in ? a.policy[at] : 0;
-      cf[tid] = in ? a.coef[at] : 0.f;
-      gm[tid] = in ? a.grm[at] : 0.f;
+      L.ctl[tid] = in ? a.policy[at] : -1;
+      L.aux[tid] = in ? a.coef[at] : 0.f;
+      L.grm[tid] = in ? a.grm[at] : 0.f;
     }
     __syncthreads();
-    int LDAy = LDA, laney = lane;
-    asm volatile("" : "+s"(LDAy), "+v"(laney));
-    // The controls some path of the tile takes this year (the same mask in
-    // every wave): only their products are formed in both sweeps below.
-    unsigned used = 0u;
-    {
-      const int cl = lane < kRovsRows ? ctl[lane] : -1;
-      for (int c = 0; c < C; ++c)
-        if (__ballot(cl == c) != 0ull) used |= 1u << c;
-    }
-    // x_t: the product under the path's control.
-#pragma unroll
-    for (int t = 0; t < NT; ++t) sel[t] = floatx16{};
-    for (int c = 0; c < C; ++c) {
-      if (!((used >> c) & 1u)) continue;
-      const PackedB B = packed_b(a.mpack + (size_t)c * Pp * a.Pk, nkg, mbytes);
-      if (my_n == 1)
-        rovs_product<TF, 1>(acc, B, A, tcol, LDAy, arow, akoff, laney);
-      else if (my_n == 2)
-        rovs_product<TF, 2>(acc, B, A, tcol, LDAy, arow, akoff, laney);
-#pragma unroll
-      for (int r = 0; r < TF::NACC; ++r) {
-        if (ctl[TF::acc_row(laney, r)] == c) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            if (t < my_n) sel[t][r] = acc[t][r];
-        }
-      }
-    }
-    __syncthreads();  // every wave has read n_t before w_t overwrites it
+    if (wave == 0) rg_group(sh, L.ctl, L.map, L.tiles, lane);
+    __syncthreads();
+    // x_t = n_t M_u.
+    rg_move<NCW>(sh, X, reinterpret_cast<const char*>(a.mpack), mbytes, L.ctl, L.map, L.tiles, wave,
+                 lane);
     // w_t = lambda_t+1 o G'(x_t) + coef_t (the growth noise drawn as the
     // forward pass drew it), into the tile and the per-control planes.
-    int LDAe = LDA, p0e = p0, lanee = lane;
-    asm volatile("" : "+s"(LDAe), "+s"(p0e), "+v"(lanee));
+    rg_quads(sh, a.cols, p0, year, a.tag0, a.key0, a.key1, wave, lane,
+             [&](int row, int col, float K, float Ki, const float* z) {
+               const float4 gm = *reinterpret_cast<const float4*>(L.grm + row);
+               const float4 cf = *reinterpret_cast<const float4*>(L.aux + row);
+               const float g[4] = {gm.x + z[0] * a.lv, gm.y + z[1] * a.lv, gm.z + z[2] * a.lv,
+                                   gm.w + z[3] * a.lv};
+               const float q[4] = {cf.x, cf.y, cf.z, cf.w};
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (t >= my_n) break;
-      const int col = tcol[t] * TF::TN + TF::acc_col(lanee);
-      const int pcol = TF::perm(col);
-      const float Kc = K[col], Ki = Kinv[col];
-      const bool real = col < a.P;
-#pragma unroll
-      for (int r4 = 0; r4 < TF::NACC; r4 += 4) {
-        float z[4];
-        const int row0 = TF::acc_row(lanee, r4);
-        TF::normal4((uint32_t)(p0e + row0) >> 2, (uint32_t)year, (uint32_t)col, a.tag0, a.key0,
-                    a.key1, z);
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const int row = TF::acc_row(lanee, r4 + s4);
-          const float x = sel[t][r4 + s4];
-          const float g = gm[row] + z[s4] * a.lv;
-          const float w =
-              real ? lam[t][r4 + s4] * (1.f + g * (Kc - 2.f * x) * Ki * 0.01f) + cf[row] : 0.f;
-          A[row * LDAe + pcol] = w;
-          const int path = p0e + row;
-          if (path < N) a.w_out[((size_t)year * N + path) * Pp + col] = w;
-        }
-      }
-    }
+               for (int s = 0; s < 4; ++s) {
+                 const int at = (row + s) * sh.LDA + col;
+                 const float x = X[at];
+                 const float w =
+                     col < a.P ? Y[at] * (1.f + g[s] * (K - 2.f * x) * Ki * 0.01f) + q[s] : 0.f;
+                 X[at] = w;
+                 const int path = p0 + row + s;
+                 if (path < N) a.w_out[((size_t)year * N + path) * Pp + col] = w;
+               }
+             });
     __syncthreads();
     // lambda_t = w_t M_u^T.
-#pragma unroll
-    for (int t = 0; t < NT; ++t) lam[t] = floatx16{};
-    for (int c = 0; c < C; ++c) {
-      if (!((used >> c) & 1u)) continue;
-      const PackedB B = packed_b(a.mtpack + (size_t)c * Pp * a.Pk, nkg, mbytes);
-      if (my_n == 1)
-        rovs_product<TF, 1>(acc, B, A, tcol, LDAy, arow, akoff, laney);
-      else if (my_n == 2)
-        rovs_product<TF, 2>(acc, B, A, tcol, LDAy, arow, akoff, laney);
-#pragma unroll
-      for (int r = 0; r < TF::NACC; ++r) {
-        if (ctl[TF::acc_row(laney, r)] == c) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            if (t < my_n) lam[t][r] = acc[t][r];
-        }
-      }
-    }
-    __syncthreads();  // every wave has read w_t before the next year's tile
+    rg_move<NCW>(sh, X, reinterpret_cast<const char*>(a.mtpack), mbytes, L.ctl, L.map, L.tiles,
+                 wave, lane);
+    float* const t = X;
+    X = Y;
+    Y = t;
   }
 }
 
@@ -1258,17 +1537,23 @@ hipError_t launch_ctl_rows(const int* ctl, int n, int C, int* blk_count, int* bl
   return hipGetLastError();
 }
 
+hipError_t launch_rovs_policy_forward(const RovsForwardArgs& a, hipStream_t s) {
+  if (a.C < 1 || a.C > kRovsMaxC || !a.rvec || a.Pp % 32 || a.Pp > kRovsMaxPatches)
+    return hipErrorInvalidValue;
+  return rg_launch(rg_plan(a.N, a.Pp, a.C, 1, 1),
+                   rg_cols(a.Pp) == 1 ? reinterpret_cast<const void*>(&rovs_policy_kernel<1>)
+                                      : reinterpret_cast<const void*>(&rovs_policy_kernel<2>),
+                   a, s);
+}
+
 hipError_t launch_rovs_adj(const RovsAdjArgs& a, hipStream_t s) {
-  if (a.N < 1 || a.T < 1 || a.C < 1 || a.C > kRovsMaxC || a.Pp % TF::TN || a.Pp > kRovsMaxPatches ||
+  if (a.N < 1 || a.T < 1 || a.C < 1 || a.C > kRovsMaxC || a.Pp % 32 || a.Pp > kRovsMaxPatches ||
       a.P > a.Pp || a.Pk % 16 || a.Pk > a.Pp || a.Pk < a.P)
     return hipErrorInvalidValue;
-  const size_t lds = rovs_adj_lds(a.Pp);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&rovs_adj_kernel),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
-  const int blocks = (a.N + kRovsRows - 1) / kRovsRows;
-  hipLaunchKernelGGL(rovs_adj_kernel, dim3(blocks), dim3(64 * rovs_waves(a.Pp)), lds, s, a);
-  return hipGetLastError();
+  return rg_launch(rg_plan(a.N, a.Pp, a.C, 2, 1),
+                   rg_cols(a.Pp) == 1 ? reinterpret_cast<const void*>(&rovs_adj_kernel<1>)
+                                      : reinterpret_cast<const void*>(&rovs_adj_kernel<2>),
+                   a, s);
 }
 
 hipError_t launch_rovs_recompute(const RovsRecomputeArgs& a, hipStream_t s) {
