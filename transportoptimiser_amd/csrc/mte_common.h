@@ -383,42 +383,6 @@ __device__ __forceinline__ void year_product(typename TR::AccT* acc,
   for (int kg = 2; kg < nkg; kg += 2) step(kg, std::false_type{});
 }
 
-// acc += A[rows of tile (trow, tcol), k-groups kg0 .. kg1) . M[those k-groups,
-// cols of the tile] for one output tile, kg1 > kg0, with the same two-stage
-// ping-pong as year_product (the operands of the next k-group are in flight
-// while the MFMAs of the current one run) and an odd tail step.
-template <class TR>
-__device__ __forceinline__ void range_product(typename TR::AccT& acc, const PackedB& B,
-                                              const typename TR::T* A, int trow,
-                                              int tcol, int kg0, int kg1,
-                                              int LDA, int arow, int akoff, int lane) {
-  using T = typename TR::T;
-  using VecT = typename TR::VecT;
-  constexpr int TM = TR::TM, KV = TR::KV;
-  const uint32_t boff = b_voff(B, tcol, lane);
-  const T* ap = A + (trow * TM + arow) * LDA + akoff;
-  VecT b0 = load_b<VecT>(B, boff, kg0);
-  VecT a0 = *reinterpret_cast<const VecT*>(ap + kg0 * 8);
-  int kg = kg0;
-  for (; kg + 1 < kg1; kg += 2) {
-    const VecT b1 = load_b<VecT>(B, boff, kg + 1);
-    const VecT a1 = *reinterpret_cast<const VecT*>(ap + (kg + 1) * 8);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int s = 0; s < KV; ++s) acc = TR::mfma(a0[s], b0[s], acc);
-    const int k2 = min(kg + 2, kg1 - 1);
-    b0 = load_b<VecT>(B, boff, k2);
-    a0 = *reinterpret_cast<const VecT*>(ap + k2 * 8);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int s = 0; s < KV; ++s) acc = TR::mfma(a1[s], b1[s], acc);
-  }
-  if (kg < kg1) {
-#pragma unroll
-    for (int s = 0; s < KV; ++s) acc = TR::mfma(a0[s], b0[s], acc);
-  }
-}
-
 // Split-bf16 form of year_product (TraitsB3).  A k-chunk is 16 k: the A
 // operands are 8 bf16 of the hi and of the lo array (Ah and Ah + lo_off), the
 // B operands packed k-groups 2c (hi) and 2c + 1 (lo).  Each chunk issues the
@@ -504,7 +468,7 @@ __device__ __forceinline__ void year_product_b3(floatx16* acc, const PackedB& B,
 }
 
 // acc += the split-bf16 product over k-chunks c0 .. c1 (c1 > c0) of one tile,
-// with range_product's ping-pong and odd tail.
+// with year_product_b3's ping-pong and an odd tail step.
 __device__ __forceinline__ void range_product_b3(floatx16& acc, const PackedB& B,
                                                  const uint16_t* Ah, int lo_off, int trow,
                                                  int tcol, int c0, int c1, int LDA, int arow,
