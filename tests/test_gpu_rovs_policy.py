@@ -29,11 +29,26 @@ pytestmark = pytest.mark.gpu
     (16, 3, 1),      # one path
 ])
 def test_groups_match_oracle(ctx, oracle, P, C, N):
-    T = 4
+    pol = np.random.default_rng(P).integers(0, C, size=(4, N)).astype(np.int32)
+    pol[1] = C - 1  # a year of one group
+    _check(ctx, oracle, P, pol, C)
+
+
+@pytest.mark.parametrize("P", [48, 300])
+def test_eight_controls_most_paths_under_one(ctx, oracle, P):
+    # Every control taken in each 32-path tile, seven of them once: eight
+    # groups, more than the row map holds.
+    pol = np.full((4, 70), 7, np.int32)
+    for t in range(4):
+        for p0 in (0, 32):
+            pol[t, p0 + np.random.default_rng([P, t, p0]).permutation(32)[:7]] = np.arange(7)
+    _check(ctx, oracle, P, pol, 8)
+
+
+def _check(ctx, oracle, P, pol, C):
+    T, N = pol.shape
     pr = rs.synthetic_problem(seed=5, n_patches=P, n_species=1, n_controls=C, n_paths=N,
                               n_years=T, threshold_ratio=0.97)
-    pol = np.random.default_rng(P).integers(0, C, size=(T, N)).astype(np.int32)
-    pol[1] = C - 1  # a year of one group
     tau = 0.02 * pr.species[0].params[3]
     print(f"grouped rows P={P} C={C} N={N}", flush=True)
     val, g = rs.smooth_value_gradient(ctx, pr, pol, tau)

@@ -37,6 +37,7 @@
 
 #include "mte_common.h"
 #include "rng.h"
+#include "rovs_group.h"
 #include "rovs_kernels.h"
 
 namespace roadmc {
@@ -987,90 +988,19 @@ hipError_t launch_rovs_smooth_value(const RovsSmoothArgs& a, hipStream_t s) {
 // At P = 256, C = 3, N = 100,000, T = 50: forward 8.8 ms, reverse
 // sweep 16.0 ms (20.7 and 34.6 ms with 32-path tiles on the FP32 MFMA, every
 // control a tile uses multiplied and each path's product selected).
-constexpr int kRgWaves = 8, kRgThreads = kRgWaves * 64;
-constexpr int kRgTiles = 7;  // group tiles at most
-constexpr int kRgMaxRows = 160;
-constexpr int kRgParts = 4;  // column quarters of a row's dots
-
-// Column tiles a wave owns, and the group tiles whose products it can hold:
-// 7 (an eighth spills in the product loop) or 4 of two columns.
-static int rg_cols(int Pp) { return Pp > 32 * kRgWaves ? 2 : 1; }
-__host__ __device__ constexpr int rg_slots(int cols) { return cols == 1 ? kRgTiles : 4; }
-
-// Group tiles that BM rows under C controls can need.
-static int rg_max_tiles(int BM, int C) { return (BM - std::min(C, BM)) / 32 + std::min(C, BM); }
-
-struct RgPlan {
-  int BM;
-  int dense;  // 32 rows, every used control's product, selected per path
-  size_t lds;
-};
-
-// LDS: n_tiles tiles, then [kRgParts][C + 1][BM] partial dots, [n_st][C + 1][BM]
-// dots, growth-rate means, totals or coefficients, controls, the row map
-// ([kRgTiles][32]) and the tiles' controls.
-static size_t rg_lds(int BM, int Pp, int C, int n_tiles, int n_st) {
-  return sizeof(float) * ((size_t)n_tiles * BM * (Pp + TraitsX6::PAD) +
-                          (size_t)(kRgParts + n_st) * (C + 1) * BM + 3 * (size_t)BM + kRgTiles * 32 + 16);
-}
-
-// The rows of a launch over N paths: of the sizes (whole path quads) that LDS
-// and the waves' registers allow, the one with the least rounds of workgroups
-// over the CUs times work, in product tiles: 1.6 for 32 paths (product, growth
-// and dots) and half a tile of padding per control.  The results do not depend
-// on the rows.
-static RgPlan rg_plan(int N, int Pp, int C, int n_tiles, int n_st) {
-  constexpr size_t kLdsMax = 160 * 1024;
-  constexpr int kCus = 256;
-  RgPlan best{32, 0, rg_lds(32, Pp, C, n_tiles, n_st)};
-  best.dense = rg_max_tiles(8, C) > rg_slots(rg_cols(Pp));
-  double cost = 1e300;
-  for (int BM = 8; BM <= kRgMaxRows; BM += 4) {
-    const size_t lds = rg_lds(BM, Pp, C, n_tiles, n_st);
-    if (lds > kLdsMax || rg_max_tiles(BM, C) > rg_slots(rg_cols(Pp))) continue;
-    const int rounds = ((N + BM - 1) / BM + kCus - 1) / kCus;
-    const double c = rounds * (1.6 * BM / 32 + 0.5 * C);
-    if (c < cost) {
-      cost = c;
-      best = RgPlan{BM, 0, lds};
-    }
-  }
-  return best;
-}
-
-struct RgShape {
-  int BM, Pp, LDA, nch, C, dense;
-};
+static_assert(kRgPad == TraitsX6::PAD, "row distance of the tile");
 
 // A fresh copy of the lane number, so that the addresses and columns derived
 // from it are computed again where they are used instead of being kept, and
 // spilled, over the year loop.
 __device__ __forceinline__ void rg_opaque(int* lane) { asm volatile("" : "+v"(*lane)); }
 
-// Wave 0: map [tile][32] holds the row of each group slot (-1 in the padding),
-// tiles[t] the control of group tile t and tiles[kRgTiles] their number.  ctl
-// is -1 for rows past the last path.
+// The row map of a year's controls, by one wave.
 __device__ __forceinline__ void rg_group(const RgShape& sh, const int* ctl, int* map, int* tiles,
                                          int lane) {
-#pragma unroll
-  for (int i = 0; i < kRgTiles * 32; i += 64)
-    if (i + lane < kRgTiles * 32) map[i + lane] = -1;
-  const int c0 = lane < sh.BM ? ctl[lane] : -1;
-  const int c1 = 64 + lane < sh.BM ? ctl[64 + lane] : -1;
-  const int c2 = 128 + lane < sh.BM ? ctl[128 + lane] : -1;
-  const uint64_t below = (1ull << lane) - 1;
-  int nt = 0;
-  for (int c = 0; c < sh.C; ++c) {
-    const uint64_t m0 = __ballot(c0 == c), m1 = __ballot(c1 == c), m2 = __ballot(c2 == c);
-    const int n0 = __popcll(m0), n1 = n0 + __popcll(m1), n = n1 + __popcll(m2);
-    if (c0 == c) map[32 * nt + __popcll(m0 & below)] = lane;
-    if (c1 == c) map[32 * nt + n0 + __popcll(m1 & below)] = 64 + lane;
-    if (c2 == c) map[32 * nt + n1 + __popcll(m2 & below)] = 128 + lane;
-    const int k = (n + 31) >> 5;
-    if (lane < k) tiles[nt + lane] = c;
-    nt += k;
-  }
-  if (lane == 0) tiles[kRgTiles] = nt;
+  rg_group_clear(sh, map, lane);
+  rg_group_fill(sh, ctl, map, tiles, lane,
+                [](int, int v, int c) -> uint64_t { return __ballot(v == c); });
 }
 
 // Replaces each path's row of the tile by its product with its control's
@@ -1289,24 +1219,6 @@ __device__ __forceinline__ void rg_store(const RgShape& sh, const float* A, floa
           *reinterpret_cast<const floatx4*>(A + r * sh.LDA + c);
 }
 
-// LDS arrays after the tiles.
-struct RgArrays {
-  float *part, *st, *grm, *aux;
-  int *ctl, *map, *tiles;
-};
-__device__ __forceinline__ RgArrays rg_arrays(const RgShape& sh, float* smem, int n_tiles,
-                                              int n_st) {
-  RgArrays r;
-  r.part = smem + (size_t)n_tiles * sh.BM * sh.LDA;
-  r.st = r.part + kRgParts * (sh.C + 1) * sh.BM;
-  r.grm = r.st + n_st * (sh.C + 1) * sh.BM;
-  r.aux = r.grm + sh.BM;
-  r.ctl = reinterpret_cast<int*>(r.aux + sh.BM);
-  r.map = r.ctl + sh.BM;
-  r.tiles = r.map + kRgTiles * 32;
-  return r;
-}
-
 template <int NCW>
 __global__ __launch_bounds__(kRgThreads) void rovs_policy_kernel(RovsForwardArgs a, int BM,
                                                                      int dense) {
@@ -1374,7 +1286,7 @@ __global__ __launch_bounds__(kRgThreads) void rovs_policy_kernel(RovsForwardArgs
 // Launches fn(args, rows, dense) over the paths.
 template <class Args>
 static hipError_t rg_launch(const RgPlan& pl, const void* fn, const Args& a, hipStream_t s) {
-  if (pl.lds > 160 * 1024) return hipErrorInvalidValue;
+  if (pl.lds > kRgLdsMax) return hipErrorInvalidValue;
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds);
   if (e != hipSuccess) return e;
   Args arg = a;
