@@ -51,7 +51,9 @@ static void group(const RgShape& sh, size_t lds, int n_tiles, int rows, int patt
     return;
   }
   const int nt = L.tiles[kRgTiles];
-  CHECK(nt >= 0 && nt <= rg_slots(rg_cols(sh.Pp)));
+  // rg_move: the waves that share a column tile split the group tiles evenly.
+  const int ntc = sh.Pp / 32, share = ntc <= kRgWaves ? kRgWaves / ntc : 1;
+  CHECK(nt >= 0 && nt <= kRgTiles && (nt + share - 1) / share <= rg_slots(rg_cols(sh.Pp)));
   std::vector<int> seen(sh.BM, 0);
   int last_c = -1, last_r = -1;
   for (int s = 0; s < kRgTiles * 32; ++s) {
@@ -80,6 +82,9 @@ int main() {
           CHECK(pl.BM >= 8 && pl.BM <= kRgMaxRows && pl.BM % 4 == 0);
           CHECK(pl.lds == rg_lds(pl.BM, Pp, C, n_tiles, 1) && pl.lds <= kRgLdsMax);
           CHECK(!pl.dense || pl.BM == 32);
+          // Every control's product only where the waves cannot hold the
+          // groups: never where two or more waves share a column tile.
+          CHECK(pl.dense == ((C == 8 && Pp > 128) || (C > 4 && Pp > 256)));
           rows_seen[pl.BM > 128 ? 2 : pl.BM > 64 ? 1 : 0] = 1;
           dense_seen |= pl.dense;
           for (int p = 0; p < 4; ++p)

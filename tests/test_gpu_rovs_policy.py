@@ -34,10 +34,10 @@ def test_groups_match_oracle(ctx, oracle, P, C, N):
     _check(ctx, oracle, P, pol, C)
 
 
-@pytest.mark.parametrize("P", [48, 300])
+@pytest.mark.parametrize("P", [48, 200, 300])
 def test_eight_controls_most_paths_under_one(ctx, oracle, P):
     # Every control taken in each 32-path tile, seven of them once: eight
-    # groups, more than the row map holds.
+    # groups, in the grouped form (48 patches) and every control's product.
     pol = np.full((4, 70), 7, np.int32)
     for t in range(4):
         for p0 in (0, 32):
