@@ -76,7 +76,7 @@ int main() {
     for (int Pp = 64; Pp <= 512; Pp += 64)
       for (int n_tiles = 1; n_tiles <= 2; ++n_tiles)
         for (int N : {1, 7, 40, 300, 5000, 9000, 20000, 30000, 100000, 1000000}) {
-          const RgPlan pl = rg_plan(N, Pp, C, n_tiles, 1);
+          const RgPlan pl = rg_plan(N, Pp, C, n_tiles, 1, 256);
           const RgShape sh{pl.BM, Pp, Pp + kRgPad, Pp / 16, C, pl.dense};
           const int pattern = -1;
           CHECK(pl.BM >= 8 && pl.BM <= kRgMaxRows && pl.BM % 4 == 0);
@@ -87,6 +87,9 @@ int main() {
           CHECK(pl.dense == ((C == 8 && Pp > 128) || (C > 4 && Pp > 256)));
           rows_seen[pl.BM > 128 ? 2 : pl.BM > 64 ? 1 : 0] = 1;
           dense_seen |= pl.dense;
+          // The plan follows the device: half the CUs take half the paths in
+          // the same rounds.
+          CHECK(rg_plan(N, Pp, C, n_tiles, 1, 128).BM == rg_plan(2 * N, Pp, C, n_tiles, 1, 256).BM);
           for (int p = 0; p < 4; ++p)
             for (int rows : {pl.BM, pl.BM - 3, 1}) group(sh, pl.lds, n_tiles, rows, p);
         }

@@ -764,7 +764,7 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
       a.ckpt = static_cast<float*>(B.ckpt.ptr) + (size_t)sp * T * N * Pp;
       a.grm_out = static_cast<float*>(B.grm.ptr) + (size_t)sp * T * N;
     }
-    RMC_HIP(ctx, roadmc::launch_rovs_policy_forward(a, s));
+    RMC_HIP(ctx, roadmc::launch_rovs_policy_forward(a, ctx->n_cu, s));
   }
 
   // The value and the coefficients dJ_p / dA.
@@ -839,7 +839,7 @@ extern "C" int roadmc_rovs_smooth_grad(roadmc_ctx* ctx, const roadmc_rovs_proble
     a.key0 = k0;
     a.key1 = k1;
     a.w_out = static_cast<float*>(G.w.ptr);
-    RMC_HIP(ctx, roadmc::launch_rovs_adj(a, s));
+    RMC_HIP(ctx, roadmc::launch_rovs_adj(a, ctx->n_cu, s));
     for (int c = 0; c < C; ++c) {
       if (total[c] == 0) {  // no path ever under c: no dependence on its survival
         std::fill(gm.begin(), gm.end(), 0.0);

@@ -58,18 +58,17 @@ inline size_t rg_lds(int BM, int Pp, int C, int n_tiles, int n_st) {
 
 // The rows of a launch over N paths: of the sizes (whole path quads) that LDS
 // and the waves' registers allow, the one with the least rounds of workgroups
-// over the CUs times work, in product tiles: 1.6 for 32 paths (product, growth
+// over the n_cu CUs times work, in product tiles: 1.6 for 32 paths (product, growth
 // and dots) and half a tile of padding per control.  The results do not depend
 // on the rows.
-inline RgPlan rg_plan(int N, int Pp, int C, int n_tiles, int n_st) {
-  constexpr int kCus = 256;
+inline RgPlan rg_plan(int N, int Pp, int C, int n_tiles, int n_st, int n_cu) {
   RgPlan best{32, 0, rg_lds(32, Pp, C, n_tiles, n_st)};
   best.dense = rg_max_tiles(8, C) > rg_capacity(Pp);
   double cost = 1e300;
   for (int BM = 8; BM <= kRgMaxRows; BM += 4) {
     const size_t lds = rg_lds(BM, Pp, C, n_tiles, n_st);
     if (lds > kRgLdsMax || rg_max_tiles(BM, C) > rg_capacity(Pp)) continue;
-    const int rounds = ((N + BM - 1) / BM + kCus - 1) / kCus;
+    const int rounds = ((N + BM - 1) / BM + n_cu - 1) / n_cu;
     const double c = rounds * (1.6 * BM / 32 + 0.5 * C);
     if (c < cost) {
       cost = c;

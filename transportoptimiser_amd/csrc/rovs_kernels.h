@@ -49,8 +49,9 @@ struct RovsForwardArgs {
 hipError_t launch_rovs_forward(const RovsForwardArgs& a, hipStream_t s);
 // The same for controls fixed by a policy: FP32 products of each path's own
 // control only; mpack is the matrices' three-term split (6 bytes an entry) and
-// the checkpoints are in patch order.
-hipError_t launch_rovs_policy_forward(const RovsForwardArgs& a, hipStream_t s);
+// the checkpoints are in patch order.  The rows of a workgroup follow n_cu, the
+// device's CUs.
+hipError_t launch_rovs_policy_forward(const RovsForwardArgs& a, int n_cu, hipStream_t s);
 
 // Unit profit per path and year: unit_cost + sum_v fuel_cost_v price_{fuel_idx_v}
 // - unit_revenue sum_c composition_c price_{n_fuels + c}.
@@ -168,7 +169,7 @@ struct RovsAdjArgs {
   uint32_t tag0, key0, key1;
   float* w_out;           // [T][N][Pp]
 };
-hipError_t launch_rovs_adj(const RovsAdjArgs& a, hipStream_t s);
+hipError_t launch_rovs_adj(const RovsAdjArgs& a, int n_cu, hipStream_t s);
 
 // Lists of the n rows of ctl [n] by control, stable.  First call (scatter
 // false): blk_count and blk_off [ceil(n / 1024)][C] and the totals [C].  Second

@@ -1449,20 +1449,20 @@ hipError_t launch_ctl_rows(const int* ctl, int n, int C, int* blk_count, int* bl
   return hipGetLastError();
 }
 
-hipError_t launch_rovs_policy_forward(const RovsForwardArgs& a, hipStream_t s) {
-  if (a.C < 1 || a.C > kRovsMaxC || !a.rvec || a.Pp % 32 || a.Pp > kRovsMaxPatches)
+hipError_t launch_rovs_policy_forward(const RovsForwardArgs& a, int n_cu, hipStream_t s) {
+  if (n_cu < 1 || a.C < 1 || a.C > kRovsMaxC || !a.rvec || a.Pp % 32 || a.Pp > kRovsMaxPatches)
     return hipErrorInvalidValue;
-  return rg_launch(rg_plan(a.N, a.Pp, a.C, 1, 1),
+  return rg_launch(rg_plan(a.N, a.Pp, a.C, 1, 1, n_cu),
                    rg_cols(a.Pp) == 1 ? reinterpret_cast<const void*>(&rovs_policy_kernel<1>)
                                       : reinterpret_cast<const void*>(&rovs_policy_kernel<2>),
                    a, s);
 }
 
-hipError_t launch_rovs_adj(const RovsAdjArgs& a, hipStream_t s) {
-  if (a.N < 1 || a.T < 1 || a.C < 1 || a.C > kRovsMaxC || a.Pp % 32 || a.Pp > kRovsMaxPatches ||
+hipError_t launch_rovs_adj(const RovsAdjArgs& a, int n_cu, hipStream_t s) {
+  if (n_cu < 1 || a.N < 1 || a.T < 1 || a.C < 1 || a.C > kRovsMaxC || a.Pp % 32 || a.Pp > kRovsMaxPatches ||
       a.P > a.Pp || a.Pk % 16 || a.Pk > a.Pp || a.Pk < a.P)
     return hipErrorInvalidValue;
-  return rg_launch(rg_plan(a.N, a.Pp, a.C, 2, 1),
+  return rg_launch(rg_plan(a.N, a.Pp, a.C, 2, 1, n_cu),
                    rg_cols(a.Pp) == 1 ? reinterpret_cast<const void*>(&rovs_adj_kernel<1>)
                                       : reinterpret_cast<const void*>(&rovs_adj_kernel<2>),
                    a, s);
