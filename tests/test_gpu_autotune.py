@@ -47,6 +47,18 @@ def test_autotune_keeps_the_fastest_valid_setting(ctx, keep_tiles, prec):
         assert ctx.tile(prec, b) == {k: chosen[0][k] for k in ("rows", "split", "per_cu")}
 
 
+def test_autotune_times_the_rows_it_names(ctx, keep_tiles):
+    # 8 x 2,048 paths are 256 workgroups of 64 rows and 64 of 256 rows, on a
+    # quarter of the CUs: four times the work in a row, so about three times the
+    # time.  Were a small trial run with fewer rows than it names, the two would
+    # be the same launch.
+    print("autotune rows with few paths", flush=True)
+    trials = ctx.autotune(n_paths=2048, n_years=40, precision=nat.PREC_FP32)
+    ms = {r: min(t["ms"] for t in trials if t["bucket_max_p"] == 128 and t["rows"] == r)
+          for r in (64, 256)}
+    assert ms[256] > 1.5 * ms[64], ms
+
+
 def test_set_tile_rejects_invalid_settings(ctx, keep_tiles):
     for args in [(nat.PREC_FP64, 128, 32, 0, 0), (nat.PREC_FP32, 100, 32, 0, 0),
                  (nat.PREC_FP32, 1024, 64, 0, 0), (nat.PREC_FP32, 256, 48, 0, 0),

@@ -36,9 +36,6 @@ struct MteJob {
 };
 
 constexpr int kMteThreads = 512;  // 8 waves per workgroup
-// FP32 workgroups of at most this many output tiles take 4 waves, two
-// workgroups to a CU where LDS allows.
-constexpr int kMteTilesFourWaves = 16;
 
 // Element budget BM*Pp of one workgroup's population tile.
 constexpr int kMteTileElemsF32 = 32768;

@@ -16,6 +16,7 @@
 #include "ctx.h"
 #include "road_host.h"
 #include "mte_kernels.h"
+#include "mte_plan.h"
 #include "rng.h"
 #include "roadmc.h"
 #include "mte_wide.h"
@@ -26,7 +27,7 @@ namespace {
 
 constexpr int kBuckets = 4;
 const int kBucketMax[kBuckets] = {128, 256, 512, 1024};
-constexpr size_t kLdsPerCu = 160 * 1024;  // gfx950 LDS per CU
+using roadmc::kMteLdsPerCu;
 
 int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
@@ -248,31 +249,23 @@ struct JobSet {
 };
 
 void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roads,
-               bool want_end_pops, JobSet& js) {
+               bool want_end_pops, bool nominal, JobSet& js) {
   js.prec = roads[0].precision;
   js.fp64 = js.prec == ROADMC_PREC_FP64;
   const bool f32 = js.prec == roadmc::kPrecF32;
-  // Rows of paths per workgroup: the tile table's; in FP32, where a path's
-  // result does not depend on them, halved (down to 32) while the launch has
-  // fewer workgroups than the card has CUs: 256 patches and 5,000 paths
-  // 1.27 -> 0.84 ms, 100 patches and 2,000 paths 0.78 -> 0.54 ms.
-  int shrink = 1;
-  auto rows_of = [&](const roadmc_mte_problem& pr, int Pp) {
-    const int granule = js.fp64 ? roadmc::kMteRowsF64 : roadmc::kMteRowsF32;
-    return std::max(granule,
-                    rows_for(ctx, js.prec, Pp, pr.n_paths) / shrink / granule * granule);
-  };
-  auto workgroups = [&]() {
-    int64_t n = 0;
-    for (int r = 0; r < n_roads; ++r)
-      for (int s = 0; s < roads[r].n_species; ++s) {
-        const int bm = rows_of(roads[r], round_up(roads[r].species[s].n_patches, 32));
-        n += (roads[r].n_paths + bm - 1) / bm;
-      }
-    return n;
-  };
-  while (f32 && shrink < 8 && workgroups() < ctx->n_cu) shrink *= 2;
-  const bool fills = workgroups() > ctx->n_cu;
+  std::vector<roadmc::MtePlanJob> pj;
+  for (int r = 0; r < n_roads; ++r)
+    for (int s = 0; s < roads[r].n_species; ++s) {
+      const int Pp = round_up(roads[r].species[s].n_patches, 32);
+      pj.push_back({Pp, roads[r].n_paths, rows_for(ctx, js.prec, Pp, roads[r].n_paths)});
+    }
+  std::vector<roadmc::MtePlanTile> tiles;
+  if (f32)
+    tiles = roadmc::mte_plan_f32(pj, ctx->n_cu, nominal, [](int rows, int Pp) {
+      return roadmc::mte_lds_bytes(roadmc::kPrecF32, rows, Pp, 0);
+    });
+  else
+    for (const auto& j : pj) tiles.push_back({j.rows, 8});
   for (int r = 0; r < n_roads; ++r) {
     const roadmc_mte_problem& pr = roads[r];
     for (int s = 0; s < pr.n_species; ++s) {
@@ -284,7 +277,7 @@ void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roa
       jb.Pk = js.prec == roadmc::kPrecB3 ? jb.Pp : round_up(jb.P, 16);
       jb.N = (int32_t)pr.n_paths;
       jb.T = pr.n_years;
-      jb.BM = rows_of(pr, jb.Pp);
+      jb.BM = tiles[js.jobs.size()].rows;
       jb.law = pr.growth_law;
       jb.endpoint = pr.endpoint;
       jb.n_tiles = (int)((pr.n_paths + jb.BM - 1) / jb.BM);
@@ -320,17 +313,9 @@ void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roa
       const int rem = ntiles % 4;
       jb.split = js.prec == roadmc::kPrecB3 && rem &&
                  ctx->tiles[tile_slot(js.prec)][bucket_of(jb.Pp)].split && (jb.Pk >> 3) >= 8 &&
-                 roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem) <= kLdsPerCu;
-      // FP32 tiles of at most 16 output tiles run as four-wave workgroups,
-      // two of them on a CU (see mte_kernels.hip); larger ones, those whose LDS
-      // leaves no room for a second and those of a launch without a second
-      // workgroup for some CU as eight-wave workgroups.
-      const int waves = f32 && fills && ntiles <= roadmc::kMteTilesFourWaves &&
-                                2 * roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, 0) <= kLdsPerCu
-                            ? 4
-                            : 8;
+                 roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem) <= kMteLdsPerCu;
+      js.waves.push_back(tiles[js.jobs.size()].waves);
       js.jobs.push_back(jb);
-      js.waves.push_back(waves);
       js.road_of.push_back(r);
       js.species_of.push_back(s);
     }
@@ -805,7 +790,7 @@ extern "C" int roadmc_mte_run(roadmc_ctx* ctx, const roadmc_mte_problem* problem
     if (problem->species[s].n_patches > ROADMC_MAX_PATCHES)
       return mte_run_wide(ctx, problem, result);
   JobSet js;
-  plan_jobs(ctx, problem, 1, result->end_pops != nullptr, js);
+  plan_jobs(ctx, problem, 1, result->end_pops != nullptr, false, js);
   JobBuffers& b = ctx->mte_bufs;
   rc = js.fp64 ? upload_jobs<double>(ctx, problem, js, b, false)
                : upload_jobs<float>(ctx, problem, js, b, false);
@@ -883,8 +868,12 @@ int capture_batch_graph(roadmc_batch* bt) {
 
 }  // namespace
 
-extern "C" int roadmc_batch_prepare(roadmc_ctx* ctx, const roadmc_mte_problem* roads,
-                                    int32_t n_roads, roadmc_batch** out) {
+namespace {
+
+// roadmc_batch_prepare; nominal: the tile table's rows whatever the batch's
+// size (mte_plan.h).
+int batch_prepare(roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roads, bool nominal,
+                  roadmc_batch** out) {
   if (!ctx) return ROADMC_ERR_INVALID;
   if (!out || !roads || n_roads < 1)
     return rmc_fail(ctx, ROADMC_ERR_INVALID, "roads/out invalid");
@@ -904,7 +893,7 @@ extern "C" int roadmc_batch_prepare(roadmc_ctx* ctx, const roadmc_mte_problem* r
   RMC_HIP(ctx, hipSetDevice(ctx->device));
   roadmc_batch* bt = new roadmc_batch();
   bt->ctx = ctx;
-  plan_jobs(ctx, roads, n_roads, true, bt->js);
+  plan_jobs(ctx, roads, n_roads, true, nominal, bt->js);
   int rc = bt->js.fp64 ? upload_jobs<double>(ctx, roads, bt->js, bt->bufs, true)
                        : upload_jobs<float>(ctx, roads, bt->js, bt->bufs, true);
   if (!rc) rc = ensure_lds_limit(ctx, bt->js.prec, bt->js.lds_max());
@@ -919,7 +908,7 @@ extern "C" int roadmc_batch_prepare(roadmc_ctx* ctx, const roadmc_mte_problem* r
             ctx->tiles[tile_slot(bt->js.prec)][bucket_of(bt->js.jobs[j].Pp)].per_cu;
         want = std::min(want, pc == 0 ? 2 : pc);
       }
-      l.grid = ctx->n_cu * ((want == 2 && l.lds * 2 <= kLdsPerCu) ? 2 : 1);
+      l.grid = ctx->n_cu * ((want == 2 && l.lds * 2 <= kMteLdsPerCu) ? 2 : 1);
     }
     bt->roads.assign(roads, roads + n_roads);
     rc = capture_batch_graph(bt);
@@ -930,6 +919,13 @@ extern "C" int roadmc_batch_prepare(roadmc_ctx* ctx, const roadmc_mte_problem* r
   }
   *out = bt;
   return ROADMC_OK;
+}
+
+}  // namespace
+
+extern "C" int roadmc_batch_prepare(roadmc_ctx* ctx, const roadmc_mte_problem* roads,
+                                    int32_t n_roads, roadmc_batch** out) {
+  return batch_prepare(ctx, roads, n_roads, false, out);
 }
 
 extern "C" int roadmc_batch_launch(roadmc_batch* bt) {
@@ -1135,10 +1131,10 @@ extern "C" int roadmc_autotune_ex(roadmc_ctx* ctx, int32_t precision, int32_t n_
       const size_t lds_max = roadmc::mte_lds_bytes(precision, rows, P, 3);
       for (int split = 0; split <= (precision == ROADMC_PREC_BF16X3 ? 1 : 0); ++split) {
         const size_t lds = split ? lds_max : roadmc::mte_lds_bytes(precision, rows, P, 0);
-        for (int per_cu = 1; per_cu <= (lds * 2 <= kLdsPerCu ? 2 : 1); ++per_cu) {
+        for (int per_cu = 1; per_cu <= (lds * 2 <= kMteLdsPerCu ? 2 : 1); ++per_cu) {
           ctx->tiles[slot][b] = {rows, split, per_cu};
           roadmc_batch* bt = nullptr;
-          int rc = roadmc_batch_prepare(ctx, prs.data(), kRoads, &bt);
+          int rc = batch_prepare(ctx, prs.data(), kRoads, true, &bt);
           double ms = 0.0;
           if (!rc) rc = roadmc_batch_launch(bt);  // warm-up
           if (!rc) rc = roadmc_batch_kernel_ms(bt, &ms);
