@@ -5,7 +5,8 @@ One year with the pre-growth endpoint returns the product itself.  With K
 terms a destination's value takes ceil(K / 8) roundings of the sum of the
 large term products and as many, 2^-8 smaller, of the small ones (each
 rounding cut by at most 2^-8 of the last place), one rounding each of the
-state, the movement entry and the final sum, and the dropped term products:
+state, its row's scale, the movement entry and the final sum, and the dropped
+term products (three below 2^-25):
 |error| <= (ceil(K / 8) (1 + 2^-6) + 6) 2^-24 of a sum of non-negative terms.
 A product without any one of the six terms exceeds it."""
 import numpy as np
@@ -66,3 +67,20 @@ def test_small_launch_takes_fewer_rows_with_the_same_bits(ctx):
         for x, y in ((a.end_pops, b.end_pops), (a.end_mean, b.end_mean), (a.end_sd, b.end_sd),
                      (a.patch_mean[0], b.patch_mean[0]), (a.mte_prob, b.mte_prob)):
             np.testing.assert_array_equal(x, y)
+
+
+def test_mean_of_nearly_equal_paths_averages_the_roundings(ctx, oracle):
+    # REF_CPU's noise is 1e-4 of a population: paths share the first bits of
+    # every entry.  A patch's mean over N paths is within the roundings common
+    # to all of them (the movement matrix's 2^-24 an entry, averaged over the
+    # destination's terms, and the populations' few FP32 constants: 1e-8 rms)
+    # and 1 / sqrt(32) of one product's rms error (1.3e-7 at 512 patches): 2.5e-8.
+    # Paths that round alike leave 7e-8.
+    rng = np.random.default_rng(7)
+    sd = ls.make_species(rng, 512)
+    pr = ls.RoadProblem([sd], n_years=8, n_paths=1024, growth_law=nat.LAW_REF_CPU, seed=4)
+    print("nearly equal paths", flush=True)
+    out = ctx.simulate_mte(pr)
+    ref = oracle.mte_problem(pr)["patch_mean"][0]
+    err = np.linalg.norm(out.patch_mean[0] - ref) / np.linalg.norm(ref)
+    assert err <= 4e-8, err

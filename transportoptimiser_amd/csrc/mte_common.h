@@ -146,6 +146,15 @@ struct TraitsB3 {
 // it is read (28 VALU operations per 8 values); the movement matrix is split
 // once when it is packed.  Operand and accumulator lane layouts are those of
 // TraitsB3.
+// The tile holds a path's populations times its row's scale, one of 32 in
+// (0.5, 1].  The sums of h.h' depend on the populations' first 8 bits only, so
+// that paths closer to each other than that (a law with little noise) would
+// round alike in every sum, and their mean would keep one path's error: 7e-8
+// of a patch's mean at 512 patches under REF_CPU, where the FP32 MFMA's larger
+// errors average to 2e-8.  Scaled, paths have different first bits whatever
+// the noise (2e-8).  The product and the growth factor commute with the scale;
+// only the level in the growth law takes its inverse, one multiplication per
+// value and year.
 struct TraitsX6 {
   using T = float;
   using VecT = floatx4;
@@ -154,6 +163,15 @@ struct TraitsX6 {
   static constexpr bool kQuadItems = true;
   static constexpr bool kSplit = false;
   __device__ static AccT mfma(floatx4 a, floatx4 b, AccT c) { return TraitsB3::mfma(a, b, c); }
+  // Inverse scale of a row, the product of the factors of its accumulator item
+  // r and of its lane half, row = acc_row(lane, r).  Exact short numbers: one
+  // that rounds would move the level of every patch of a row alike (5e-10 of
+  // the mean total a year).
+  __host__ __device__ static constexpr float unscale(int row) {
+    return (float)((32 + 2 * ((row >> 1 & 12) | (row & 3))) * (32 + (row >> 2 & 1))) / 1024.f;
+  }
+  __device__ static constexpr float unscale_item(int r) { return (float)(32 + 2 * r) / 32.f; }
+  __device__ static float unscale_half(int lane) { return lane < 32 ? 1.f : 33.f / 32.f; }
   __device__ static int acc_row(int lane, int r) {
     return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
   }
@@ -229,16 +247,17 @@ __host__ __device__ static inline size_t lds_bytes_t(int BM, int Pp, int n_rem_s
          (size_t)n_rem_split * 4 * TR::NACC * 64 * sizeof(T);
 }
 
+// n' = level grown by a year, times x / level.
 template <typename T, int LAW>
-__device__ __forceinline__ T grow(T x, T z, T K, T Kinv, T r, T sig,
+__device__ __forceinline__ T grow(T x, T level, T z, T K, T Kinv, T r, T sig,
                                   T half_var, T dt, T mu, T sd, T grm, T lv) {
   if constexpr (LAW == kLawRefCpu) {
     const T g = dt * (mu + sd * z) * (T)0.01;
-    return x * ((T)1 + g * (K - x) * Kinv);
+    return x * ((T)1 + g * (K - level) * Kinv);
   }
   if constexpr (LAW == kLawRefGpu) {
     const T g = lv * z * grm + grm;
-    return x * ((T)1 + g * (K - x) * Kinv);
+    return x * ((T)1 + g * (K - level) * Kinv);
   }
   T e;
   if constexpr (sizeof(T) == 4)
@@ -246,7 +265,7 @@ __device__ __forceinline__ T grow(T x, T z, T K, T Kinv, T r, T sig,
     e = __builtin_amdgcn_exp2f(fmaf(sig, z, -half_var));
   else
     e = exp(sig * z - half_var);
-  return x * ((T)1 + r * ((T)1 - x * Kinv)) * e;
+  return x * ((T)1 + r * ((T)1 - level * Kinv)) * e;
 }
 
 template <typename T>

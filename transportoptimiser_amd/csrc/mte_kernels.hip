@@ -44,6 +44,15 @@ size_t mte_lds_bytes(int prec, int BM, int Pp, int n_rem_split) {
 }
 
 
+// Inverse scales of the 32 rows of a block (TraitsX6).
+struct RowUnscale {
+  double v[32];
+  constexpr RowUnscale() : v() {
+    for (int r = 0; r < 32; ++r) v[r] = (double)TraitsX6::unscale(r);
+  }
+};
+__device__ constexpr RowUnscale kRowUnscale;
+
 // Simulates one tile (BM paths of one job) for all years and writes the
 // tile's tallies.  Every thread of the workgroup calls it.  The growth law is
 // a template parameter so that the epilogue has no per-element branches.
@@ -96,6 +105,8 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       const uint32_t hl = TR::split(init[c]);
       Ah[r * LDA + c] = (uint16_t)hl;
       Ah[lo_off + r * LDA + c] = (uint16_t)(hl >> 16);
+    } else if constexpr (kX6) {
+      A[r * LDA + c] = init[c] / TR::unscale(r);
     } else {
       A[r * LDA + TR::perm(c)] = init[c];
     }
@@ -196,7 +207,9 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       RMC_GLOBAL T* ck = gmem(static_cast<T*>(jb.ckpt)) + ((size_t)(year / jb.ckpt_every) * jb.N) * Pp;
       for (int idx = tid; idx < BM * Pp; idx += nthreads) {
         const int r = idx / Pp, c = idx - r * Pp;
-        if (p0 + r < jb.N) ck[(size_t)(p0 + r) * Pp + c] = A[r * LDA + TR::perm(c)];
+        T v = A[r * LDA + TR::perm(c)];
+        if constexpr (kX6) v *= TR::unscale(r);
+        if (p0 + r < jb.N) ck[(size_t)(p0 + r) * Pp + c] = v;
       }
     }
     if constexpr (TR::kSplit) {
@@ -346,6 +359,10 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
     const T sig_y = (kFastLn && keep_pre) ? (T)0 : sig;
     const T hv_y = (kFastLn && keep_pre) ? (T)0 : half_var;
     const T rscale = (kFastLn && keep_pre) ? (T)0 : (T)1;
+    // The level of a scaled population x: x times its item's and its half's
+    // inverse (1 where nothing is scaled).
+    T unhalf = (T)1;
+    if constexpr (kX6) unhalf = TR::unscale_half(lanee);
     auto store = [&](const int row, const int pc, const T v) {
       if constexpr (TR::kSplit) {
         const uint32_t hl = TR::split(v);
@@ -360,7 +377,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       const int col = tc * TN + TR::acc_col(lanee);
       const int pcol = TR::perm(col);
       const T K = colse[col], Ki = colse[Pp + col], rr = colse[2 * Pp + col];
-      const T ga = (T)1 + rr * rscale, gb = rr * rscale * Ki;
+      const T ga = (T)1 + rr * rscale, gb = rr * rscale * Ki * unhalf;
 #pragma unroll
       for (int r4 = 0; r4 < NACC; r4 += 4) {
         if (kX6 && NT == 1 && r4 * parts / NACC != share) continue;
@@ -383,14 +400,16 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
             zz = z[path & 3u];
           }
           const T x = a[r4 + s];
+          T unitem = (T)1;
+          if constexpr (kX6) unitem = TR::unscale_item(r4 + s);
           if constexpr (kFastLn) {
             const T e = __builtin_amdgcn_exp2f(fmaf(sig_y, zz, -hv_y));
-            store(row, pcol, x * fmaf(-gb, x, ga) * e);
+            store(row, pcol, x * fmaf(-(gb * unitem), x, ga) * e);
           } else {
             T g = (T)0;
             if constexpr (LAW == kLawRefGpu) g = grm[row];
-            const T n = grow<T, LAW>(x, zz, K, Ki, rr, sig, half_var, dt, mu,
-                                     sd, g, lv);
+            const T n = grow<T, LAW>(x, x * (unhalf * unitem), zz, K, Ki, rr, sig, half_var,
+                                     dt, mu, sd, g, lv);
             store(row, pcol, keep_pre ? x : n);
           }
         }
@@ -436,6 +455,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       if (path < jb.N) {
         double tot = 0.0;
         for (int c = 0; c < Pp; ++c) tot += state_at(tid, c);
+        tot *= (double)TR::unscale(tid);
         if (jb.end_pops) gmem(jb.end_pops)[path] = tot;
         v[0] = tot >= jb.thr_total ? 1.0 : 0.0;
         v[1] = tot;
@@ -452,7 +472,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       const int rb = i / Pp, c = i - rb * Pp;
       const int n = min(32, jb.N - p0 - 32 * rb);
       double s = 0.0;
-      for (int r = 0; r < n; ++r) s += state_at(32 * rb + r, c);
+      for (int r = 0; r < n; ++r) s += state_at(32 * rb + r, c) * kRowUnscale.v[r];
       if (n > 0) part0[(size_t)rb * (3 + Pp) + 3 + c] = s;
     }
     __syncthreads();  // LDS is reused by the next tile
@@ -837,13 +857,13 @@ __global__ void mte_plain_kernel(PlainArgs a) {
       const T x = nxt[k];
       const T Ki = (T)1 / caps[k];
       if (a.law == kLawRefCpu)
-        cur[k] = grow<T, kLawRefCpu>(x, z, caps[k], Ki, rates[k], sig, half_var, dt, prm[1],
+        cur[k] = grow<T, kLawRefCpu>(x, x, z, caps[k], Ki, rates[k], sig, half_var, dt, prm[1],
                                      prm[2], grm, prm[7]);
       else if (a.law == kLawRefGpu)
-        cur[k] = grow<T, kLawRefGpu>(x, z, caps[k], Ki, rates[k], sig, half_var, dt, prm[1],
+        cur[k] = grow<T, kLawRefGpu>(x, x, z, caps[k], Ki, rates[k], sig, half_var, dt, prm[1],
                                      prm[2], grm, prm[7]);
       else
-        cur[k] = grow<T, kLawLognormal>(x, z, caps[k], Ki, rates[k], sig, half_var, dt,
+        cur[k] = grow<T, kLawLognormal>(x, x, z, caps[k], Ki, rates[k], sig, half_var, dt,
                                         prm[1], prm[2], grm, prm[7]);
     }
   }

@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void mte_wide_year_kernel(MteWideArgs a) {
             float g = 0.f;
             if constexpr (LAW == kLawRefGpu) g = gmem(a.grm)[n];
             v = a.keep_pre ? x
-                           : grow<float, LAW>(x, z[s], K, Ki, rr, a.sig, a.half_var, a.dt, a.mu,
+                           : grow<float, LAW>(x, x, z[s], K, Ki, rr, a.sig, a.half_var, a.dt, a.mu,
                                               a.sd, g, a.lv);
           }
           out[(size_t)n * Pp + col] = live ? v : 0.f;
