@@ -6,6 +6,8 @@ too); FP64 kernels within 1e-10; the MTE
 probability may differ only through paths that sit within that tolerance of
 the threshold.  Batched and single-road launches are bit-identical.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -323,3 +325,24 @@ def test_config2_full_size(ctx):
             thr = np.median(ref.end_pops[:, s])
             d = abs(np.mean(o.end_pops[:, s] >= thr) - np.mean(ref.end_pops[:, s] >= thr))
             assert d <= 2e-3
+
+
+def test_prepared_fp32_batch_keeps_one_copy_of_its_matrices(ctx):
+    # 12 roads of 1,024 patches: 6 bytes an entry for the split matrices (72 MiB);
+    # the FP32 packing they come from (48 MiB) is given back.  Paths, results and
+    # allocation granules stay below 16 MiB.
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert nat.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0  # libroadmc's runtime
+        return free.value
+
+    sp = make_species(np.random.default_rng(3), 1024)
+    roads = [RoadProblem([sp], n_years=1, n_paths=64, road_id=i) for i in range(12)]
+    print("memory of a prepared batch", flush=True)
+    ctx.prepare_batch(roads).close()  # the context's own scratch
+    before = free_bytes()
+    with ctx.prepare_batch(roads) as b:
+        b.launch()
+        b.sync()
+        used = before - free_bytes()
+    assert 0 < used <= (72 + 16) << 20, used

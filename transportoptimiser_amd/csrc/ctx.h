@@ -16,7 +16,7 @@ struct rmc_devbuf {
 
 struct rmc_job_buffers {
   // mpack: the packed movement matrices as uploaded or built; mx6: their
-  // three-term split (FP32 launches).
+  // three-term split (FP32 launches), after which a prepared batch frees its mpack.
   rmc_devbuf mpack, mx6, cols, partial, out, endpop, jobs, work, off, counter;
 };
 
