@@ -9,11 +9,12 @@
 //
 // How this file computes it: the paths of one species form an [N x P] state
 // matrix and a year is the product [N x P] . [P x P] followed by an
-// elementwise epilogue.  One workgroup (8 waves) owns BM paths for all T
-// years:
-//   - the BM x P population tile stays in LDS for the whole simulation, with
-//     the k index permuted inside groups of 8 so that a lane's MFMA A operands
-//     for 4 consecutive k-steps are one 16-byte LDS read;
+// elementwise epilogue.  One workgroup (8 waves; 4 for FP32 tiles of up to 16
+// output tiles) owns BM paths for all T years:
+//   - the BM x P population tile stays in LDS for the whole simulation, k in
+//     natural order in the FP32 and split-bf16 forms, whose A operands are 8
+//     consecutive k, and permuted in FP64 (TraitsF64::perm) so that a lane's
+//     operands for consecutive k-steps are one LDS read;
 //   - R is pre-packed in MFMA B-operand order, so each wave's B load is one
 //     coalesced 1 KB read that L2 serves to every workgroup of the road;
 //   - FP32 products run as six bf16 term products (TraitsX6, FP32 accumulate)
@@ -119,7 +120,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   // be even is each SIMD's, not each wave's.
   //  - Without splitting: wave w takes a contiguous run of ceil or floor of
   //    ntiles / NW tiles.
-  //  - With splitting (jb.split): each SIMD takes q = ntiles / 4 whole tiles,
+  //  - With splitting (jb.split, split bf16 only): each SIMD takes q = ntiles / 4 whole tiles,
   //    shared evenly by its waves, and each of the ntiles % 4 remaining tiles
   //    is cut into four k-quarters, quarter s going to the last wave of SIMD
   //    s.  The quarters meet in LDS, where the last wave of SIMD i sums the
@@ -128,9 +129,10 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   const int ntc = Pp / TN;
   const int ntiles = (BM / TM) * ntc;
   const int simd = wave & 3, nth = wave >> 2;
+  const bool split = TR::kSplit && jb.split;
   const bool pieces = nth == NW / 4 - 1;  // takes the k-quarter pieces
   int my_n, my_t0, n_rem = 0, q4 = 0;
-  if (jb.split) {
+  if (split) {
     q4 = ntiles >> 2;
     n_rem = ntiles & 3;
     const int base = q4 / (NW / 4), extra = q4 % (NW / 4);
@@ -418,7 +420,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
 #pragma unroll
     for (int t = 0; t < NT; ++t)
       if (t < my_n) epilogue(acc[t], trow[t], tcol[t]);
-    if (pieces && simd < n_rem) {
+    if (split && pieces && simd < n_rem) {
       // Remainder tile `simd`: the four quarters in order, then its epilogue.
       AccT sum = AccT{};
       const T* slot = qpart + (size_t)(simd * 4 * NACC) * 64 + lanee;
