@@ -93,6 +93,17 @@ int main() {
           for (int p = 0; p < 4; ++p)
             for (int rows : {pl.BM, pl.BM - 3, 1}) group(sh, pl.lds, n_tiles, rows, p);
         }
+  // The rows that the GPU test's sizes are meant to reach.
+  const int reach[][5] = {{33001, 64, 3, 132, 132}, {39985, 64, 8, 160, 160},
+                          {20005, 128, 7, 80, 80},  {30011, 192, 3, 120, 60},
+                          {33003, 256, 2, 132, 68}, {10011, 320, 2, 40, 40}};
+  for (const auto& r : reach)
+    for (int n_tiles = 1; n_tiles <= 2; ++n_tiles) {
+      const RgPlan pl = rg_plan(r[0], r[1], r[2], n_tiles, 1, 256);
+      const RgShape sh{pl.BM, r[1], r[1] + kRgPad, r[1] / 16, r[2], pl.dense};
+      const int pattern = -1;
+      CHECK(pl.BM == r[2 + n_tiles] && !pl.dense);
+    }
   printf("%s: rows up to 64 %d, 128 %d, 160 %d, dense %d, failures %d\n",
          failures ? "FAILED" : "ok", rows_seen[0], rows_seen[1], rows_seen[2], dense_seen,
          failures);

@@ -70,12 +70,16 @@ def test_set_tile_rejects_invalid_settings(ctx, keep_tiles):
 
 def _roads():
     # One road per bucket (P = 100, 200, 300, 700 patches); P = 200 and 300
-    # leave remainder tiles at 32 rows, so the split setting matters.
+    # leave remainder tiles at 32 rows, so the split setting matters,
     out = []
     for i, P in enumerate((100, 200, 300, 700)):
         sp = landscape.make_species(np.random.default_rng(50 + i), P, mort_max=0.4,
                                     threshold_ratio=0.7)
         out.append(landscape.RoadProblem([sp], n_years=6, n_paths=1000, seed=9, road_id=i))
+    # and one of 70,000 paths, so that the batch has more workgroups than CUs at
+    # any rows (an FP32 launch with fewer takes fewer rows than it is set to).
+    sp = landscape.make_species(np.random.default_rng(60), 24)
+    out.append(landscape.RoadProblem([sp], n_years=1, n_paths=70000, seed=9, road_id=9))
     return out
 
 
@@ -101,7 +105,10 @@ def test_rows_and_per_cu_do_not_change_results(ctx, keep_tiles, prec):
             np.testing.assert_array_equal(a, e)
         for a, e in zip(base_mte, mte):
             np.testing.assert_array_equal(a, e)
-    # the k-split of remainder tiles: FP32 rounding only
+    # the k-split of remainder tiles (split bf16; FP32 has none): rounding only
     ends, _ = _run(ctx, roads, prec, lambda b: 32, 1, 1)
     for a, e in zip(base, ends):
-        np.testing.assert_allclose(e, a, rtol=2e-6)
+        if prec == nat.PREC_FP32:
+            np.testing.assert_array_equal(e, a)
+        else:
+            np.testing.assert_allclose(e, a, rtol=2e-6)

@@ -18,8 +18,8 @@ from transportoptimiser_amd import native as nat
 pytestmark = pytest.mark.gpu
 
 # Patch counts around the 16-term chunks, the 32-wide tiles and the waves'
-# shares; path counts that make one, two, three (single row tiles) and more
-# row tiles, whole and ragged.
+# shares.  Alone and in a batch of one road, these path counts leave CUs idle:
+# 32-row tiles of eight waves, whole and ragged.
 SIZES = [1, 15, 16, 17, 31, 33, 48, 64, 65, 96, 130, 160, 200, 257, 300, 416, 512, 700, 1024]
 
 
@@ -48,6 +48,49 @@ def test_one_year_product_within_the_fp32_bound(ctx, N):
             err = np.abs(out.patch_mean[0] - ref) / ref
             assert err.max() <= bound, (P, err.max(), bound)
             np.testing.assert_allclose(out.end_pops[:, 0], ref.sum(), rtol=bound)
+
+
+def _filler():
+    # 70,000 paths of 20 patches: more workgroups than CUs at any rows, so that
+    # every road of the batch takes the tile table's rows.
+    return ls.RoadProblem([ls.make_species(np.random.default_rng(81), 20)], n_years=1,
+                          n_paths=70000, seed=2, road_id=99)
+
+
+@pytest.fixture
+def keep_tiles(ctx):
+    saved = ctx.tile_table(nat.PREC_FP32)
+    yield
+    for b, t in saved.items():
+        ctx.set_tile(nat.PREC_FP32, b, t["rows"], t["split"], t["per_cu"])
+
+
+# Path counts that make one, two, three, five and seven row tiles (an odd number
+# has no 2 x 2 blocks, and a wave's run of tiles crosses row blocks) and whole
+# workgroups; rows of 32 to 256, four-wave workgroups (up to 16 output tiles) and
+# eight-wave ones (17 to 32).
+@pytest.mark.parametrize("rows", [32, 64, 128, 256])
+def test_tiles_of_a_full_launch_within_the_fp32_bound(ctx, keep_tiles, rows):
+    for b in (128, 256, 512, 1024):
+        ctx.set_tile(nat.PREC_FP32, b, min(rows, 32768 // b), 0, 0)
+    roads = []
+    for P in (1, 17, 48, 64, 96, 128, 130, 200, 256, 300, 416, 512, 700, 1024):
+        for N in (32, 70, 150, 220, 256, 300):
+            roads.append(_road(P, N, 3))
+            roads[-1].road_id = len(roads)
+    print(f"{len(roads)} roads at {rows} rows", flush=True)
+    batch = ctx.simulate_mte_batch(roads + [_filler()], end_pops=True)
+    for pr, out in zip(roads, batch):
+        sd, P = pr.species[0], pr.species[0].n_patches
+        ref = (sd.init_pop[:, None] * sd.trans * sd.surv).sum(0)
+        bound = (-(-P // 8) * (1 + 2.0 ** -6) + 6) * 2.0 ** -24
+        err = np.abs(out.patch_mean[0] - ref) / ref
+        assert err.max() <= bound, (P, pr.n_paths, err.max(), bound)
+        np.testing.assert_allclose(out.end_pops[:, 0], ref.sum(), rtol=bound)
+        if rows > 32:  # the same bits as in 32-row tiles, which a road alone takes
+            one = ctx.simulate_mte(pr)
+            np.testing.assert_array_equal(out.end_pops, one.end_pops)
+            np.testing.assert_array_equal(out.patch_mean[0], one.patch_mean[0])
 
 
 def test_small_launch_takes_fewer_rows_with_the_same_bits(ctx):

@@ -1,8 +1,10 @@
 """The policy kernels of the smoothed gradient group a workgroup's paths by
 control: the sizes where the grouping changes form (column tiles shared by the
 waves, one or two per wave; every control's product above 256 patches with
-more than four controls or up to 256 with eight; path counts that are no whole
-quads or tiles), against the FP64 oracle on the same streams.
+more than four controls or above 128 with eight; path counts that are no whole
+quads or tiles; few paths, which take 8 rows a workgroup or 32 in the form of
+every control, and many, which take up to 160), against the FP64 oracle on the
+same streams.
 
 Bounds: the FP32 state of T years carries T roundings of at most 2^-23 per
 product and growth step and the survival matrices one of 2^-24; the smoothed
@@ -19,11 +21,13 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("P,C,N", [
-    (32, 8, 37),     # eight controls: every control's product
-    (40, 7, 150),    # two column tiles, four waves each; seven groups at most
-    (96, 2, 33),     # three column tiles, two idle waves
+    (32, 8, 37),     # two column tiles, four waves each; eight groups of 8 rows
+    (40, 7, 150),    # seven groups at most
+    (96, 2, 33),     # four column tiles, two waves each
+    (160, 3, 41),    # six column tiles, two idle waves
     (250, 4, 261),   # eight column tiles, a partial one
-    (257, 3, 70),    # two column tiles for one wave
+    (250, 8, 37),    # every control's product
+    (257, 3, 70),    # two column tiles for some waves
     (300, 5, 41),    # every control's product, two column tiles
     (512, 4, 45),    # the most patches
     (16, 3, 1),      # one path
@@ -31,6 +35,25 @@ pytestmark = pytest.mark.gpu
 def test_groups_match_oracle(ctx, oracle, P, C, N):
     pol = np.random.default_rng(P).integers(0, C, size=(4, N)).astype(np.int32)
     pol[1] = C - 1  # a year of one group
+    _check(ctx, oracle, P, pol, C)
+
+
+# Rows of a workgroup in the forward pass and the reverse sweep as the plan
+# chooses them on 256 CUs (tests/native/rovs_group_check.cpp holds it to them):
+# groups over 32 rows and pairs of row tiles, rows in the second and third
+# ballot, dots over several 64-row groups, a last workgroup of few paths.
+@pytest.mark.parametrize("P,C,N", [
+    (40, 3, 33001),   # 132 and 132
+    (40, 8, 39985),   # 160 and 160: twelve group tiles at most
+    (100, 7, 20005),  # 80 and 80
+    (130, 3, 30011),  # 120 and 60, six column tiles: two idle waves
+    (200, 2, 33003),  # 132 and 68
+    (257, 2, 10011),  # 40 and 40, two column tiles for some waves
+])
+def test_many_paths_match_oracle(ctx, oracle, P, C, N):
+    pol = np.random.default_rng(P).integers(0, C, size=(3, N)).astype(np.int32)
+    pol[1] = 0  # one group of all rows
+    pol[2, : N // 2] = C - 1  # workgroups of one group beside mixed ones
     _check(ctx, oracle, P, pol, C)
 
 
