@@ -167,8 +167,11 @@ void roadmc_batch_destroy(roadmc_batch* batch);
  * left after an even share per SIMD) be computed as four k-quarters, 0 not
  * (the FP32 kernels never do);
  * per_cu 1 or 2 workgroups per CU of the persistent launch (0: two when LDS
- * allows; a batch takes the smallest of its buckets' values).
- * An FP32 launch with fewer workgroups than CUs takes fewer rows.
+ * allows; a launch takes the smallest of its buckets' values.  An FP32 batch
+ * runs its tiles of up to 16 output tiles of 32 x 32 and its larger ones as two
+ * launches side by side, any other batch is one launch).
+ * An FP32 launch with fewer workgroups than CUs takes fewer rows than set,
+ * except in the tuner's trials.
  * Rows and per_cu never change results (each path's products and draws are
  * the same in any tile); a split changes the k-summation order of the split
  * tiles' paths, so their end totals move within FP32 rounding.

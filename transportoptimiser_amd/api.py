@@ -226,6 +226,9 @@ class Context:
 
     def set_tile(self, precision: int, bucket_max_p: int, rows: int, split: int = 1,
                  per_cu: int = 0) -> None:
+        """``roadmc_set_tile``: the tile setting of a patch-count bucket.
+        ``split`` has no effect in FP32, whose kernels never split, and an FP32
+        launch with fewer workgroups than CUs takes fewer rows than set."""
         nat.check(nat.lib().roadmc_set_tile(self.handle, precision, bucket_max_p, rows, split,
                                             per_cu), self.handle)
 
