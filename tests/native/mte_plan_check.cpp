@@ -48,6 +48,15 @@ int main() {
   CHECK(f[1].rows == 256 && f[1].waves == 8);
   CHECK(f[2].rows == 32 && f[2].waves == 4);
   CHECK(f[3].rows == 32 && f[3].waves == 8);
+  // Row scales: for noise that is there and small.
+  const double prm[8] = {0.05, 0.05, 0.1, 0.5, 0.5, 0.05, 0.1, 0.2}, zero[8] = {};
+  CHECK(!mte_low_noise(ROADMC_LAW_LOGNORMAL, 1.0, 0.0, prm));
+  CHECK(mte_low_noise(ROADMC_LAW_LOGNORMAL, 1.0, 0.001, prm));
+  CHECK(!mte_low_noise(ROADMC_LAW_LOGNORMAL, 1.0, 0.1, prm));
+  CHECK(mte_low_noise(ROADMC_LAW_REF_CPU, 1.0, 0.0, prm));
+  CHECK(!mte_low_noise(ROADMC_LAW_REF_CPU, 1.0, 0.1, zero));
+  CHECK(mte_low_noise(ROADMC_LAW_REF_GPU, 1.0, 0.0, prm));
+  CHECK(!mte_low_noise(ROADMC_LAW_REF_GPU, 1.0, 0.1, zero));
   printf("%s\n", failures ? "FAILED" : "ok");
   return failures ? 1 : 0;
 }

@@ -127,3 +127,21 @@ def test_mean_of_nearly_equal_paths_averages_the_roundings(ctx, oracle):
     ref = oracle.mte_problem(pr)["patch_mean"][0]
     err = np.linalg.norm(out.patch_mean[0] - ref) / np.linalg.norm(ref)
     assert err <= 4e-8, err
+
+
+@pytest.mark.parametrize("law", [nat.LAW_LOGNORMAL, nat.LAW_REF_CPU, nat.LAW_REF_GPU])
+def test_unchanged_populations_keep_their_exact_total(ctx, law):
+    # Nothing moves, dies, grows or varies: a product with the identity adds one
+    # exact term to zeros, so every path ends at its initial total exactly and
+    # meets a threshold of all of it.
+    for P in (1, 20, 100):
+        cap = 10.0 + 7.0 * np.arange(P)
+        sd = ls.SpeciesData(trans=np.eye(P), surv=np.ones((P, P)), init_pop=3.0 + np.arange(P),
+                            capacity=cap, growth=np.zeros(P), params=np.zeros(8), noise_sd=0.0,
+                            threshold_ratio=1.0)
+        pr = ls.RoadProblem([sd], n_years=5, n_paths=300, growth_law=law)
+        print(f"unchanged populations law={law} P={P}", flush=True)
+        for out in (ctx.simulate_mte(pr), ctx.simulate_mte_batch([pr], end_pops=True)[0]):
+            np.testing.assert_array_equal(out.end_pops[:, 0], sd.init_pop.sum())
+            np.testing.assert_array_equal(out.patch_mean[0], sd.init_pop)
+            assert out.mte_prob[0] == 1.0

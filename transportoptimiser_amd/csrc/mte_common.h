@@ -147,15 +147,15 @@ struct TraitsB3 {
 // it is read (28 VALU operations per 8 values); the movement matrix is split
 // once when it is packed.  Operand and accumulator lane layouts are those of
 // TraitsB3.
-// The tile holds a path's populations times its row's scale, one of 32 in
-// (0.5, 1].  The sums of h.h' depend on the populations' first 8 bits only, so
-// that paths closer to each other than that (a law with little noise) would
-// round alike in every sum, and their mean would keep one path's error: 7e-8
-// of a patch's mean at 512 patches under REF_CPU, where the FP32 MFMA's larger
-// errors average to 2e-8.  Scaled, paths have different first bits whatever
-// the noise (2e-8).  The product and the growth factor commute with the scale;
-// only the level in the growth law takes its inverse, one multiplication per
-// value and year.
+// The tile of a job with little noise (MteJob::scaled) holds a path's
+// populations times its row's scale, one of 32 in (0.5, 1].  The sums of h.h'
+// depend on the populations' first 8 bits only, so that paths closer to each
+// other than that would round alike in every sum, and their mean would keep one
+// path's error: 7e-8 of a patch's mean at 512 patches under REF_CPU, where the
+// FP32 MFMA's larger errors average to 2e-8.  Scaled, paths have different first
+// bits whatever the noise (1.3e-8).  The product and the growth factor commute
+// with the scale; only the level in the growth law takes its inverse, one
+// multiplication per value and year.
 struct TraitsX6 {
   using T = float;
   using VecT = floatx4;

@@ -32,6 +32,7 @@ struct MteJob {
   int32_t Pk;          // contraction extent: P rounded up to 16 (<= Pp); Pp
                        // in the split-bf16 form (an even count of 16-k chunks)
   int32_t split;       // split the ntiles % 4 remainder tiles into k-quarters
+  int32_t scaled;      // FP32: rows scaled (TraitsX6), set by mte_low_noise
   uint32_t tag0, tag1, key0, key1;
 };
 

@@ -61,7 +61,8 @@ __device__ constexpr RowUnscale kRowUnscale;
 // tiles are allocated whether or not a wave uses them, so the launch picks the
 // smallest form that holds its jobs' tiles, which leaves registers for more
 // resident workgroups.  NW is the workgroup's waves.
-template <class TR, int LAW, int NT, int NW>
+// SCALED: the rows' scales of TraitsX6 (jb.scaled).
+template <class TR, int LAW, int NT, int NW, bool SCALED>
 __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
                                              char* smem) {
   using T = typename TR::T;
@@ -106,10 +107,10 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       const uint32_t hl = TR::split(init[c]);
       Ah[r * LDA + c] = (uint16_t)hl;
       Ah[lo_off + r * LDA + c] = (uint16_t)(hl >> 16);
-    } else if constexpr (kX6) {
-      A[r * LDA + c] = init[c] / TR::unscale(r);
     } else {
-      A[r * LDA + TR::perm(c)] = init[c];
+      T v = init[c];
+      if constexpr (SCALED) v /= TR::unscale(r);
+      A[r * LDA + TR::perm(c)] = v;
     }
   }
   for (int r = tid; r < BM; r += nthreads) grm[r] = (T)jb.params[0];
@@ -210,7 +211,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       for (int idx = tid; idx < BM * Pp; idx += nthreads) {
         const int r = idx / Pp, c = idx - r * Pp;
         T v = A[r * LDA + TR::perm(c)];
-        if constexpr (kX6) v *= TR::unscale(r);
+        if constexpr (SCALED) v *= TR::unscale(r);
         if (p0 + r < jb.N) ck[(size_t)(p0 + r) * Pp + c] = v;
       }
     }
@@ -362,9 +363,9 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
     const T hv_y = (kFastLn && keep_pre) ? (T)0 : half_var;
     const T rscale = (kFastLn && keep_pre) ? (T)0 : (T)1;
     // The level of a scaled population x: x times its item's and its half's
-    // inverse (1 where nothing is scaled).
+    // inverse scale (1 where nothing is scaled).
     T unhalf = (T)1;
-    if constexpr (kX6) unhalf = TR::unscale_half(lanee);
+    if constexpr (SCALED) unhalf = TR::unscale_half(lanee);
     auto store = [&](const int row, const int pc, const T v) {
       if constexpr (TR::kSplit) {
         const uint32_t hl = TR::split(v);
@@ -403,7 +404,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
           }
           const T x = a[r4 + s];
           T unitem = (T)1;
-          if constexpr (kX6) unitem = TR::unscale_item(r4 + s);
+          if constexpr (SCALED) unitem = TR::unscale_item(r4 + s);
           if constexpr (kFastLn) {
             const T e = __builtin_amdgcn_exp2f(fmaf(sig_y, zz, -hv_y));
             store(row, pcol, x * fmaf(-(gb * unitem), x, ga) * e);
@@ -457,7 +458,7 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       if (path < jb.N) {
         double tot = 0.0;
         for (int c = 0; c < Pp; ++c) tot += state_at(tid, c);
-        tot *= (double)TR::unscale(tid);
+        if constexpr (SCALED) tot *= (double)TR::unscale(tid);
         if (jb.end_pops) gmem(jb.end_pops)[path] = tot;
         v[0] = tot >= jb.thr_total ? 1.0 : 0.0;
         v[1] = tot;
@@ -474,7 +475,8 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
       const int rb = i / Pp, c = i - rb * Pp;
       const int n = min(32, jb.N - p0 - 32 * rb);
       double s = 0.0;
-      for (int r = 0; r < n; ++r) s += state_at(32 * rb + r, c) * kRowUnscale.v[r];
+      for (int r = 0; r < n; ++r)
+        s += SCALED ? state_at(32 * rb + r, c) * kRowUnscale.v[r] : state_at(32 * rb + r, c);
       if (n > 0) part0[(size_t)rb * (3 + Pp) + 3 + c] = s;
     }
     __syncthreads();  // LDS is reused by the next tile
@@ -517,13 +519,24 @@ __device__ __forceinline__ void mte_tile_law(const MteJob& jb, const int tile,
   __syncthreads();  // LDS is reused by the next tile
 }
 
+template <class TR, int NT, int NW, bool SCALED>
+__device__ __forceinline__ void mte_tile_scaled(const MteJob& jb, const int tile, char* smem) {
+  switch (jb.law) {
+    case kLawRefCpu: mte_tile_law<TR, kLawRefCpu, NT, NW, SCALED>(jb, tile, smem); break;
+    case kLawRefGpu: mte_tile_law<TR, kLawRefGpu, NT, NW, SCALED>(jb, tile, smem); break;
+    default: mte_tile_law<TR, kLawLognormal, NT, NW, SCALED>(jb, tile, smem); break;
+  }
+}
+
 template <class TR, int NT, int NW>
 __device__ __forceinline__ void mte_tile(const MteJob& jb, const int tile, char* smem) {
-  switch (jb.law) {
-    case kLawRefCpu: mte_tile_law<TR, kLawRefCpu, NT, NW>(jb, tile, smem); break;
-    case kLawRefGpu: mte_tile_law<TR, kLawRefGpu, NT, NW>(jb, tile, smem); break;
-    default: mte_tile_law<TR, kLawLognormal, NT, NW>(jb, tile, smem); break;
+  if constexpr (std::is_same<TR, TraitsX6>::value) {
+    if (jb.scaled) {
+      mte_tile_scaled<TR, NT, NW, true>(jb, tile, smem);
+      return;
+    }
   }
+  mte_tile_scaled<TR, NT, NW, false>(jb, tile, smem);
 }
 
 // Two waves per SIMD: one workgroup of eight waves, or two of four (FP32

@@ -311,6 +311,7 @@ void plan_jobs(const roadmc_ctx* ctx, const roadmc_mte_problem* roads, int n_roa
       // result does not depend on the tile's rows or waves.
       const int ntiles = (jb.BM / roadmc::kMteRowsF32) * (jb.Pp / 32);
       const int rem = ntiles % 4;
+      jb.scaled = f32 && roadmc::mte_low_noise(pr.growth_law, pr.time_step, sp.noise_sd, sp.params);
       jb.split = js.prec == roadmc::kPrecB3 && rem &&
                  ctx->tiles[tile_slot(js.prec)][bucket_of(jb.Pp)].split && (jb.Pk >> 3) >= 8 &&
                  roadmc::mte_lds_bytes(js.prec, jb.BM, jb.Pp, rem) <= kMteLdsPerCu;
@@ -1497,6 +1498,8 @@ extern "C" int roadmc_mte_adjoint_fwd(roadmc_ctx* ctx, const roadmc_mte_problem*
   jb.Pp = round_up(jb.P, 64);  // the gradient GEMM works in 64 x 64 blocks
   jb.Pk = jb.Pp;               // the adjoint kernels contract over Pp
   jb.split = 0;
+  jb.scaled = !adj->fp64 && roadmc::mte_low_noise(ROADMC_LAW_LOGNORMAL, pr->time_step, sp.noise_sd,
+                                                  sp.params);
   jb.N = (int32_t)pr->n_paths;
   jb.T = pr->n_years;
   // FP32: 32-row tiles.  The segment kernels hold one tile per workgroup, and
