@@ -38,7 +38,7 @@ struct roadmc_ctx {
   };
   // FP32 rows make 16 output tiles up to P = 512, so that two workgroups of
   // four waves share a CU (8 roads of 257 to 512 patches, 20,000 paths, 3
-  // years: 1.19 to 1.20 ms, against 1.25 to 1.28 with 64 rows of eight waves).
+  // years: 1.15 to 1.20 ms, against 1.25 to 1.28 with 64 rows of eight waves).
   TileSetting tiles[2][4] = {{{128, 0, 0}, {64, 0, 0}, {32, 0, 0}, {32, 0, 0}},
                              {{256, 1, 0}, {128, 1, 0}, {64, 1, 0}, {32, 1, 0}}};
   rmc_job_buffers mte_bufs;

@@ -985,8 +985,8 @@ hipError_t launch_rovs_smooth_value(const RovsSmoothArgs& a, hipStream_t s) {
 // The valuations keep the FP32 MFMA of every control: their backward passes
 // amplify the populations' last digits (a changed neighbour set or decision
 // moved the value by up to 2%), which the smoothed value does not.
-// At P = 256, C = 3, N = 100,000, T = 50: forward 9.0 ms, reverse
-// sweep 16.3 ms (20.7 and 34.6 ms with 32-path tiles on the FP32 MFMA, every
+// At P = 256, C = 3, N = 100,000, T = 50: forward 8.8 to
+// 9.0 ms, reverse sweep 16.0 to 16.3 ms (20.7 and 34.6 ms with 32-path tiles on the FP32 MFMA, every
 // control a tile uses multiplied and each path's product selected).
 // Plan, LDS layout and grouping: rovs_group.h.
 static_assert(kRgPad == TraitsX6::PAD, "row distance of the tile");
