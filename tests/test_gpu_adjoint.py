@@ -34,6 +34,19 @@ def test_adjoint_matches_oracle(ctx, oracle, prec, rtol):
     np.testing.assert_allclose(gr, grr, rtol=rtol, atol=rtol * np.abs(grr).max())
 
 
+@pytest.mark.parametrize("P", [40, 300])
+def test_adjoint_of_little_noise_matches_oracle(ctx, oracle, P):
+    # The forward pass holds its rows scaled; checkpoints are the populations.
+    # 13 years of 4 roundings of 2^-24, the sums over paths and years 1e-6.
+    pr = _problem(P, 90, 13, prec=nat.PREC_FP32, strong=True)
+    pr.species[0].noise_sd = 0.002
+    J, gm, gr = mte_gradient(ctx, pr, checkpoint_every=4)
+    Jr, gmr, grr = oracle.mte_adjoint(pr.species[0], 0, 13, 90, pr.seed)
+    assert J == pytest.approx(Jr, rel=5e-6)
+    assert np.abs(gm - gmr).max() <= 5e-6 * np.abs(gmr).max()
+    assert np.abs(gr - grr).max() <= 5e-6 * np.abs(grr).max()
+
+
 def test_checkpoint_interval_does_not_change_gradient(ctx):
     pr = _problem(64, 200, 17)
     a = mte_gradient(ctx, pr, checkpoint_every=4)

@@ -145,3 +145,29 @@ def test_unchanged_populations_keep_their_exact_total(ctx, law):
             np.testing.assert_array_equal(out.end_pops[:, 0], sd.init_pop.sum())
             np.testing.assert_array_equal(out.patch_mean[0], sd.init_pop)
             assert out.mte_prob[0] == 1.0
+
+
+@pytest.mark.parametrize("rows", [64, 256])
+def test_scaled_rows_match_oracle_in_any_tile(ctx, oracle, keep_tiles, rows):
+    # Jobs with little noise hold their rows scaled: every law, both endpoints,
+    # ragged tiles of four and eight waves.  T years carry 3 roundings of 2^-24
+    # each beside the product's bound, and the growth's noise constants 1e-6.
+    for b in (128, 256, 512, 1024):
+        ctx.set_tile(nat.PREC_FP32, b, min(rows, 32768 // b), 0, 0)
+    roads, T = [], 6
+    for P, N in ((1, 40), (33, 150), (128, 220), (200, 70), (300, 100), (600, 50)):
+        for law in (nat.LAW_LOGNORMAL, nat.LAW_REF_CPU, nat.LAW_REF_GPU):
+            for end in (nat.END_POST_GROWTH, nat.END_PRE_GROWTH):
+                sd = ls.make_species(np.random.default_rng(P), P, noise_sd=0.002)
+                roads.append(ls.RoadProblem([sd], n_years=T, n_paths=N, growth_law=law,
+                                            endpoint=end, seed=6, road_id=len(roads)))
+    print(f"{len(roads)} roads of little noise at {rows} rows", flush=True)
+    for pr, out in zip(roads, ctx.simulate_mte_batch(roads + [_filler()], end_pops=True)):
+        P = pr.species[0].n_patches
+        ref = oracle.mte_problem(pr)
+        bound = T * ((-(-P // 8) * (1 + 2.0 ** -6) + 9) * 2.0 ** -24) + 1e-6
+        np.testing.assert_allclose(out.end_pops, ref["end_pops"], rtol=bound)
+        np.testing.assert_allclose(out.patch_mean[0], ref["patch_mean"][0], rtol=bound)
+        one = ctx.simulate_mte(pr)  # 32-row tiles
+        np.testing.assert_array_equal(out.end_pops, one.end_pops)
+        np.testing.assert_array_equal(out.patch_mean[0], one.patch_mean[0])
